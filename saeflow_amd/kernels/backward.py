@@ -32,6 +32,7 @@ def csr_transpose(indptr, indices, n_cols):
     M = indptr.numel() - 1
     nnz = indices.numel()
     dev = _lib.require_gpu(("indptr", indptr), ("indices", indices))
+    indptr, indices = indptr.contiguous(), indices.contiguous()
     lib = _lib.load()
     colptr = torch.empty(n_cols + 1, dtype=torch.int64, device=dev)
     rows = torch.empty(nnz, dtype=torch.int32, device=dev)
@@ -76,7 +77,10 @@ def sparse_backward(x, W_enc, b_enc, W_dec, b_dec, csr, grad_x_hat=None, grad_va
         s = _lib.stream(dev)
         g = torch.zeros(M, D, dtype=dt, device=dev) if grad_x_hat is None else _rows(grad_x_hat, dt)
         Wd = _rows(W_dec, dt)
-        gv = None if grad_values is None else grad_values.reshape(-1)
+        # the kernels read these as dense arrays; the gradient of a sum arrives as a view that
+        # expands one element (stride 0)
+        indptr, indices, values, b_dec = (t.contiguous() for t in (indptr, indices, values, b_dec))
+        gv = None if grad_values is None else grad_values.reshape(-1).contiguous()
         if gv is not None and gv.numel() != nnz:
             raise ValueError(f"grad_values has {gv.numel()} entries for nnz={nnz}")
         # per-feature sums over the CSC

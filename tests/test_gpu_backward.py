@@ -399,3 +399,20 @@ def test_sparse_backward_feature_lengths_around_the_thresholds(dtype, D, N):
     assert int(unused.sum()) > 0
     assert torch.count_nonzero(got.W_enc.cpu()[:, unused]) == 0 and torch.count_nonzero(got.W_dec.cpu()[unused]) == 0
     assert torch.count_nonzero(got.b_enc.cpu()[unused]) == 0
+
+
+def test_sparse_backward_takes_vectors_that_are_views():
+    """The gradient of values.sum() reaches the backward as one element expanded over the CSR
+    entries (stride 0), and a caller's vectors may be strided views: the same gradients, bit for
+    bit, as from dense copies."""
+    p, x, sae = make(96, 64, 300, "relu", torch.float32, seed=5)
+    xg = x.cuda()
+    csr = saeflow_amd.encode_sparse(sae, xg)
+    G = torch.randn(96, 64, generator=torch.Generator().manual_seed(6)).cuda()
+    h = torch.full((1,), 0.25, device="cuda").expand(csr[1].numel())
+    spread = [torch.stack([t, torch.full_like(t, 7)], dim=1)[:, 0] for t in (*csr, sae.b_dec)]
+    assert h.stride() == (0,) and all(t.stride() == (2,) for t in spread)
+    want = sparse_backward(xg, sae.W_enc, sae.b_enc, sae.W_dec, sae.b_dec, csr, G, torch.full_like(csr[2], 0.25))
+    got = sparse_backward(xg, sae.W_enc, sae.b_enc, sae.W_dec, spread[3], spread[:3], G, h)
+    for name in ("W_enc", "b_enc", "W_dec", "b_dec", "x", "pre"):
+        assert torch.equal(getattr(got, name), getattr(want, name)), name
