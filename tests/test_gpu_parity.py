@@ -195,6 +195,20 @@ def test_persistent_encode_random_whole_tile_problems():
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_fused_encode_odd_d_in_of_a_padded_transposed_weight(dtype):
+    """A d_in-contiguous W_enc whose rows are padded to 16 B and end inside a dword (odd d_in in 16
+    bits): the last d_in element of every feature counts, the last feature of a tile included."""
+    M, d_in, d_sae = 3, 777, 300
+    back = torch.zeros(d_sae, 784, dtype=dtype)
+    back[:, d_in - 1] = torch.arange(1, d_sae + 1).to(dtype)
+    x = torch.zeros(M, d_in, dtype=dtype)
+    x[:, d_in - 1] = 1
+    zeros = lambda n: torch.zeros(n, dtype=dtype, device="cuda")  # noqa: E731
+    got = fused_encode(x.cuda(), back.cuda().T[:d_in], zeros(d_sae), zeros(d_in))
+    assert torch.equal(got.cpu(), back[:, d_in - 1].expand(M, d_sae))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_fused_encode_strided_weights(dtype):
     # column-major W_enc (test_kernels.py:47-52): the K-contiguous MFMA path
     p = make_params(48, 80, "relu", dtype)
