@@ -67,7 +67,10 @@ SF_API const char* sf_last_error(void);
  * tile_cfg: NULL (tuned table) or int32[6] {BLOCK_M, BLOCK_N, BLOCK_K, GROUP_M, NUM_WAVES,
  *           GROUP_N} naming one of the compiled tilings (encode.py:104 `config=`, whose Triton
  *           configs carry num_warps likewise): {256, 256, BK, G, 8 or 4, GN} or
- *           {256, 128, BK/2, G, 4, GN}, BK = 64 (16-bit W) or 32 (fp32 W), G >= 1, GN >= 0.
+ *           {256, 128, BK/2, G, 4, GN}, BK = 64 (16-bit W) or 32 (fp32 W), G >= 1, GN >= 0, or,
+ *           for a W contiguous along one axis, the small tiles {32 | 64 | 96, 64, BK, G, 2, GN},
+ *           {128, 64, BK, G, 4, GN}, {128, 128, BK/2, G, 4, GN}, {32 | 64, 128, BK, G, 4, GN} and
+ *           (rows of W 16-B aligned) {128 | 160, 256, BK, G, 4, GN}.
  *           Tile order: GN > 0 walks runs of GN feature tiles, token tile by token tile;
  *           GN = 0 walks runs of G token tiles, feature tile by feature tile (the reference's
  *           GROUP_M order, encode.py:44-52). The order changes speed only, never results.
@@ -114,7 +117,8 @@ SF_API int sf_encode_noalloc(const void* x, int64_t sxm, int64_t sxk, int x_dt,
  * kernel keeps x' in registers (encode.py:72). */
 SF_API int sf_encode_workspace_size(int64_t M, int64_t K, int w_dt, int64_t* bytes);
 
-/* Tiling the tuned table picks for sf_encode at this shape: writes
+/* Default tiling of sf_encode (a call without tile_cfg runs a small tile in its place where that is
+ * estimated to be faster; the results are the same bits): writes
  * {BLOCK_M, BLOCK_N, BLOCK_K, GROUP_M, NUM_WAVES, GROUP_N} to cfg_out (int32[6]). Mirrors
  * best_config() (encode.py:142-144), which reports the autotuner's pick. */
 SF_API int sf_encode_config(int64_t M, int64_t N, int64_t K, int w_dt, int32_t* cfg_out);
@@ -132,8 +136,7 @@ SF_API int sf_encode_config(int64_t M, int64_t N, int64_t K, int w_dt, int32_t* 
  *   - the TopK select f.topk(k) in ops._topk (reference ops.py:12-16), with sf_rows_topk and
  *     a floor no larger than each row's k-th largest value (NaN values are kept whatever
  *     the floor, as they rank above every value in the top-k).
- * Arguments as sf_encode; only the 256x256 tiling with 8 waves (tile_cfg NULL or {256, 256,
- * BLOCK_K, GROUP_M, 8, GROUP_N}). 0 <= cap <= 4096 (SF_EINVAL otherwise): sf_rows_to_csr and
+ * Arguments as sf_encode; tile_cfg NULL, {256, 256, BLOCK_K, GROUP_M, 8, GROUP_N} or a small tile. 0 <= cap <= 4096 (SF_EINVAL otherwise): sf_rows_to_csr and
  * sf_rows_topk read lists of at most 4096 entries.
  */
 SF_API int sf_encode_rows(const void* x, int64_t sxm, int64_t sxk, int x_dt,

@@ -1,9 +1,10 @@
 // Fused SAE encoder on gfx950 MFMA: entry points (C ABI) and the x' prologue launch.
 // Reference semantics: saeflow/kernels/encode.py:36-91 (kernel) and :97-139 (wrapper). The
 // kernels and their design are described in encode_kernels.h.
+#include <cmath>
 #include <mutex>
 
-#include "encode_kernels.h"
+#include "encode_slim.h"
 
 namespace sfenc {
 
@@ -97,6 +98,65 @@ extern "C" int sf_encode_workspace_size(int64_t M, int64_t K, int w_dt, int64_t*
 
 namespace {
 
+// The slim kernels' W path (encode_slim.h): the DMA paths where the 256x256 kernels have one,
+// else registers for a W that is contiguous along one axis; -1 for other strides.
+int slim_w(int wp, int64_t swk, int64_t swn) {
+  if (wp != W_GENERIC) return wp == W_NMAJOR ? S_NMAJOR : S_KMAJOR;
+  return swn == 1 ? S_NROWS : (swk == 1 ? S_KROWS : -1);
+}
+
+template <int DT>
+hipError_t launch_slim_dt(const GemmArgs& a, int sw, int shape, int epi, hipStream_t s) {
+  switch (sw) {
+    case S_NMAJOR: return launch_slim<DT, S_NMAJOR>(a, shape, epi, s);
+    case S_KMAJOR: return launch_slim<DT, S_KMAJOR>(a, shape, epi, s);
+    case S_NROWS: return launch_slim<DT, S_NROWS>(a, shape, epi, s);
+    default: return launch_slim<DT, S_KROWS>(a, shape, epi, s);
+  }
+}
+
+// The slim shape a call without a tile_cfg runs, or -1 for the 256x256 tiles: the smallest of the
+// estimated times below. A tile costs `tile` us of a CU's time once several share it and `alone` us
+// on an idle CU (K-step latencies), both measured on MI355X at d_in 2304 (16-bit) and 768 (fp32) and
+// proportional to d_in; slim tiles of a CU overlap, 256x256 tiles come in whole rounds. A call with
+// one token tile is also one pass over W at `pass` bytes per us, which hides most of the shorter of
+// the two. Measured (us a call, both sides with the x' launch): bf16 d_in 2304 d_sae 16384, 1 token
+// 53 -> 21 (32x64), 137 tokens 54 -> 30, 384 tokens 55 -> 47, from 512 tokens on 256x256 wins; d_sae
+// 65536, 1 token 63 -> 53 (32x128), 137 tokens row lists 102 -> 87 (160x256); fp32 d_in 768, 1 token
+// of d_sae 12288 185 -> 23, 300 tokens 187 -> 57; an odd d_sae of 10007, d_in 1000, 1000 tokens 143
+// (element-wise staging) -> 57.
+int pick_slim(int64_t M, int64_t N, int64_t K, int w_dt, int sw) {
+  if (sw < 0 || K == 0) return -1;
+  struct Cost {
+    float tile, alone;
+  };
+  static constexpr Cost c16[SLIM_SHAPES] = {{7.5f, 9.5f},   {10.5f, 12.5f}, {12.5f, 16.5f}, {14.f, 14.5f}, {23.f, 25.f},
+                                            {10.7f, 12.5f}, {15.f, 14.5f},  {46.f, 36.f},   {44.f, 41.f}};
+  static constexpr Cost c32[SLIM_SHAPES] = {{8.f, 10.f},  {13.7f, 22.f}, {21.f, 34.f},  {24.3f, 24.f}, {47.f, 43.f},
+                                            {13.4f, 14.f}, {24.f, 23.f},  {100.f, 92.f}, {124.f, 115.f}};
+  const bool f32 = w_dt == SF_F32, dma = sw == S_NMAJOR || sw == S_KMAJOR;
+  const double cus = 8 * XCD_CUS, pass = 5.7e6, scale = (double)K / (f32 ? 768 : 2304);
+  auto estimate = [&](double mfma, int64_t tiles_m) {
+    const double bytes = tiles_m == 1 ? (double)N * K * sf_dtype_size(w_dt) / pass : 0;
+    return std::max(mfma, bytes) + 0.25 * std::min(mfma, bytes);
+  };
+  const int64_t wm = (M + BM - 1) / BM, wn = (N + BN - 1) / BN;
+  int best = -1;
+  // (a W staged element by element: never the 256x256 tiles)
+  double least = dma ? estimate(std::ceil(wm * wn / cus) * (f32 ? 173 : 45) * scale, wm) : 1e300;
+  for (int i = 0; i < (dma ? SLIM_SHAPES : SLIM_DMA_ONLY); ++i) {
+    const SlimShape q = slim_shape(i);
+    const int64_t tm = (M + q.tm - 1) / q.tm, tn = (N + q.tn - 1) / q.tn;
+    const Cost c = f32 ? c32[i] : c16[i];
+    const double t = estimate(std::max((double)c.alone, tm * tn / cus * c.tile) * scale, tm);
+    if (t < least) {
+      least = t;
+      best = i;
+    }
+  }
+  return best;
+}
+
 template <int DT>
 hipError_t launch_rows_o(int out_dt, bool floor, const GemmArgs& a, int wp, hipStream_t s) {
   switch (out_dt) {
@@ -141,20 +201,27 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
   const int bk = bk_of(w_dt);
   int group_m = DEFAULT_GROUP_M, group_n = DEFAULT_GROUP_N, waves = DEFAULT_WAVES;
   bool wide = true;
+  int slim = -1;  // a slim shape (encode_slim.h) instead of the 256x256 and 256x128 tiles
   if (tile_cfg) {
+    for (int i = 0; i < SLIM_SHAPES && !gather; ++i) {
+      const SlimShape q = slim_shape(i);
+      if (tile_cfg[0] == q.tm && tile_cfg[1] == q.tn && tile_cfg[2] == q.kc * bk / 8 && tile_cfg[4] == q.nw) slim = i;
+    }
     const bool is_wide = tile_cfg[0] == BM && tile_cfg[1] == BN && tile_cfg[2] == bk &&
                          (tile_cfg[4] == SF_WIDE_WAVES || (tile_cfg[4] == 4 && epi == EPI_DENSE));
     const bool is_narrow = epi == EPI_DENSE && tile_cfg[0] == t2::BM && tile_cfg[1] == t2::BN &&
                            tile_cfg[2] == bk / 2 && tile_cfg[4] == 4;
-    SF_REQUIRE((is_wide || is_narrow) && tile_cfg[3] >= 1 && tile_cfg[5] >= 0,
+    SF_REQUIRE((is_wide || is_narrow || slim >= 0) && tile_cfg[3] >= 1 && tile_cfg[5] >= 0,
                "%s: unsupported tile config {%d,%d,%d,%d,%d,%d}; compiled tilings: "
-               "{%d,%d,%d,GROUP_M>=1,%d%s,GROUP_N>=0}%s", fn, tile_cfg[0], tile_cfg[1], tile_cfg[2], tile_cfg[3],
+               "{%d,%d,%d,GROUP_M>=1,%d%s,GROUP_N>=0}%s and the small {32|64|96,64,BLOCK_K,G,2,GN}, "
+               "{128,64,BLOCK_K,G,4,GN}, {128,128,BLOCK_K/2,G,4,GN}, {32|64,128,BLOCK_K,G,4,GN}, "
+               "{128|160,256,BLOCK_K,G,4,GN}", fn, tile_cfg[0], tile_cfg[1], tile_cfg[2], tile_cfg[3],
                tile_cfg[4], tile_cfg[5], BM, BN, bk, SF_WIDE_WAVES, epi == EPI_DENSE ? " or 4" : "",
                epi == EPI_DENSE ? " and {256,128,BLOCK_K/2,GROUP_M>=1,4,GROUP_N>=0}" : "");
     group_m = tile_cfg[3];
     group_n = tile_cfg[5];
     waves = tile_cfg[4];
-    wide = is_wide;
+    wide = !is_narrow;
   }
   if (epi != EPI_DENSE) {
     SF_REQUIRE(cap >= 0 && cap <= SF_ROWS_CAP_MAX, "%s: capacity %lld out of range [0, %d]", fn, (long long)cap,
@@ -189,12 +256,32 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
   a.thr = thr; a.thr_dt = act == SF_ACT_JUMPRELU ? thr_dt : SF_F32;
   a.out = out; a.som = som; a.son = son; a.out_dt = out_dt;
   a.row_nnz = row_nnz; a.M = M; a.N = N; a.K = K; a.act = act;
-  const int tbm = wide ? BM : t2::BM, tbn = wide ? BN : t2::BN;
+
+  // W layouts the DMA paths take; anything else is staged through registers
+  int wp = W_GENERIC;
+  if (swn == 1 && swk >= N && (N % epc) == 0 && ((swk * esz) % 16) == 0 && aligned(w, 16) &&
+      (int64_t)bk * swk * esz + N * esz < (1LL << 31))
+    wp = W_NMAJOR;
+  // (K * esz a multiple of 4: a buffer load drops the dword that the range ends inside, which would
+  // lose the last d_in element of a tile's last feature)
+  else if (swk == 1 && swn >= K && ((swn * esz) % 16) == 0 && aligned(w, 16) && ((K * esz) % 4) == 0 &&
+           (int64_t)BN * swn * esz + K * esz < (1LL << 31))
+    wp = W_KMAJOR;
+  const int sw = slim_w(wp, swk, swn);
+  if (tile_cfg == nullptr && !gather) slim = pick_slim(M, N, K, w_dt, sw);
+  SF_REQUIRE(slim < 0 || sw == S_NMAJOR || sw == S_KMAJOR || (sw >= 0 && slim < SLIM_DMA_ONLY),
+             "%s: the small tilings need W contiguous along one axis (those of 256 features also 16-B aligned rows)", fn);
+
+  const int tbm = slim >= 0 ? slim_shape(slim).tm : (wide ? BM : t2::BM);
+  const int tbn = slim >= 0 ? slim_shape(slim).tn : (wide ? BN : t2::BN);
   // K-steps of the chosen tiling: whole pipeline rounds (2 wide steps of bk, 3 narrow steps of
-  // bk/2) covering K; the workspace is padded for both (padded_k), so no zero round is added
-  // to the wide kernel where K is not a multiple of 384 (e.g. d_in = 4096: 64 steps, not 66)
-  const int64_t round_k = wide ? 2 * bk : 3 * (bk / 2);
-  a.ksteps = (int)((K + round_k - 1) / round_k * round_k / (wide ? bk : bk / 2));
+  // bk/2, single small-tile steps) covering K; the workspace is padded for all (padded_k), so no
+  // zero round is added to the wide kernel where K is not a multiple of 384 (e.g. d_in = 4096: 64
+  // steps, not 66)
+  const int64_t step_k = slim >= 0 ? bk * slim_shape(slim).kc / 8 : (wide ? bk : bk / 2);
+  const int64_t round_k = slim >= 0 ? step_k : (wide ? 2 * step_k : 3 * step_k);
+  a.ksteps = (int)((K + round_k - 1) / round_k * round_k / step_k);
+  if (slim >= 0) a.ksteps = std::max(a.ksteps, 1);
   a.tiles_m = (int)((M + tbm - 1) / tbm);
   a.tiles_n = (int)((N + tbn - 1) / tbn);
   // a group wider than the panels there are orders the tiles as one that covers them all (and
@@ -209,17 +296,6 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
   a.n_live = n_live;
   a.live_off = live_off;
   a.tile_ctr = (int32_t*)((char*)workspace + xw_bytes(M, K, w_dt));
-
-  // W layouts the DMA paths take; anything else is staged element-wise
-  int wp = W_GENERIC;
-  if (swn == 1 && swk >= N && (N % epc) == 0 && ((swk * esz) % 16) == 0 && aligned(w, 16) &&
-      (int64_t)bk * swk * esz + N * esz < (1LL << 31))
-    wp = W_NMAJOR;
-  // (K * esz a multiple of 4: a buffer load drops the dword that the range ends inside, which would
-  // lose the last d_in element of a tile's last feature)
-  else if (swk == 1 && swn >= K && ((swn * esz) % 16) == 0 && aligned(w, 16) && ((K * esz) % 4) == 0 &&
-           (int64_t)BN * swn * esz + K * esz < (1LL << 31))
-    wp = W_KMAJOR;
 
   hipStream_t s = (hipStream_t)stream;
   hipError_t e;
@@ -253,7 +329,13 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
     default: e = launch_xprep<SF_F32>(x, sxm, sxk, x_dt, b_dec, bdec_dt, M, K, Kp, (char*)workspace, a.tile_ctr, s); break;
   }
   if (e != hipSuccess) return sf_fail(SF_EHIP, "%s: prologue launch failed: %s", fn, hipGetErrorString(e));
-  if (epi == EPI_DENSE) {
+  if (slim >= 0) {
+    switch (w_dt) {
+      case SF_BF16: e = launch_slim_dt<SF_BF16>(a, sw, slim, epi, s); break;
+      case SF_F16: e = launch_slim_dt<SF_F16>(a, sw, slim, epi, s); break;
+      default: e = launch_slim_dt<SF_F32>(a, sw, slim, epi, s); break;
+    }
+  } else if (epi == EPI_DENSE) {
     switch (w_dt) {
       case SF_BF16: e = launch_gemm<SF_BF16>(a, wp, wide, waves, s); break;
       case SF_F16: e = launch_gemm<SF_F16>(a, wp, wide, waves, s); break;

@@ -79,7 +79,9 @@ def _autotune(key, launch, w_dtype, row_nnz, dev):
     if key not in _tuned:
         saved = row_nnz.clone() if row_nnz is not None else None
         stream = torch.cuda.current_stream(dev)  # the stream the launches go to
-        cands = _candidates(w_dtype)
+        # None: the library's own choice, which may be a small tile (ragged shapes, a W_enc whose
+        # rows are not 16-B aligned)
+        cands = [*_candidates(w_dtype), None]
         for cfg in cands:
             launch(cfg)
         events = [[] for _ in cands]
@@ -163,9 +165,12 @@ def fused_encode(x, W_enc, b_enc, b_dec, threshold=None, activation="relu", *,
       (counted on the stored, rounded values).
     config: dict {BLOCK_M, BLOCK_N, BLOCK_K, GROUP_M, NUM_WAVES, GROUP_N} naming a compiled
       tiling: {256, 256, 64 (32 for fp32), G, 8 or 4, GN} (256x256 tiles of 8 waves of 128x64
-      or 4 waves of 128x128) or {256, 128, 32 (16), G, 4, GN} (two workgroups per CU), and its
+      or 4 waves of 128x128) or {256, 128, 32 (16), G, 4, GN} (two workgroups per CU), or a small
+      tile {32 | 64 | 96, 64, 64 (32), G, 2, GN}, {128, 64, 64 (32), G, 4, GN}, {128, 128, 32 (16),
+      G, 4, GN}, {32 | 64, 128, 64 (32), G, 4, GN}, {128 | 160, 256, 64 (32), G, 4, GN}, and its
       tile order: runs of GN feature tiles if GN > 0, else runs of G token tiles (GN 0, the
-      default of a dict without it); None = autotuned.
+      default of a dict without it); None = autotuned, or, for problems too small to time, the
+      256x256 tile or a small one by an estimate of both.
     allow_tf32: accepted for compatibility; gfx950 has no xf32 matrix path, so fp32 inputs
       always run the IEEE fp32 MFMA path.
     """
@@ -206,8 +211,8 @@ def encode_rows(x, W_enc, b_enc, b_dec, threshold=None, activation="relu", *, ca
     values (the nonzeros fused_encode would store) as (column, value) pairs in
     cand_idx/cand_val[m, :min(cnt, cap)], in no particular order; cand_cnt[m] counts them
     all, so cand_cnt[m] > cap flags an overflowed row. row_floor (float32 [M], relu only)
-    keeps only stored values >= row_floor[m]. Same fused kernel as fused_encode, 256x256
-    tiling only.
+    keeps only stored values >= row_floor[m]. Same fused kernels as fused_encode: the
+    256x256 tiling with 8 waves and the small tiles.
     """
     if activation not in ACTIVATIONS:
         raise ValueError(f"encode_rows supports {list(ACTIVATIONS)}, got {activation!r}")
@@ -297,6 +302,6 @@ def encode_gather(x, W_enc, b_enc, b_dec, rows, n_rows, threshold=None, activati
 def best_config():
     """Tiling chosen by the most recent launch that chose one, i.e. a call without `config`
     (None until such a call): the autotuner's timed pick for that shape, or the default
-    tiling of a problem too small to time (encode.py:142-144). Calls that pin `config` leave
-    it unchanged."""
+    tiling of a problem too small to time (encode.py:142-144), which stands for the small tile
+    that such a problem may run instead (same bits). Calls that pin `config` leave it unchanged."""
     return None if _last_config is None else dict(_last_config)

@@ -1,0 +1,140 @@
+"""GPU: the encode's small tiles (32 to 128 tokens by 64 or 128 features) against its 256x256 tile.
+
+All tilings run the same MFMA chain per output, so features, row counts and candidate lists agree
+bit for bit with the 256x256 tile's, which the parity tests check against the oracle. Shapes end
+inside a tile, a K-step, a 16-B chunk and a 32-token block; W_enc is feature-contiguous or
+d_in-contiguous, with 16-B aligned rows (LDS DMA) or rows of odd length (staged through
+registers)."""
+
+import pytest
+import torch
+
+from saeflow_amd.kernels import encode_pre, encode_rows, fused_encode
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float32, torch.bfloat16, torch.float16]
+TILES = [(32, 64, 2), (64, 64, 2), (96, 64, 2), (128, 64, 4), (128, 128, 4), (32, 128, 4), (64, 128, 4),
+         (128, 256, 4), (160, 256, 4)]
+# (tokens, d_in, d_sae): one of everything; exact tiles; remainders on every axis; a long K loop
+SHAPES = [(1, 1, 1), (32, 64, 64), (33, 40, 72), (95, 200, 264), (97, 72, 1000), (128, 128, 128), (129, 16, 136),
+          (300, 777, 520), (5, 2304, 4096), (257, 1024, 328)]
+
+
+def config(tile, dtype):
+    tm, tn, nw = tile
+    bk = (32 if dtype == torch.float32 else 64) // (2 if (tm, tn) == (128, 128) else 1)
+    return {"BLOCK_M": tm, "BLOCK_N": tn, "BLOCK_K": bk, "GROUP_M": 1, "NUM_WAVES": nw, "GROUP_N": 4}
+
+
+def wide(dtype):
+    return {"BLOCK_M": 256, "BLOCK_N": 256, "BLOCK_K": 32 if dtype == torch.float32 else 64}
+
+
+def make(shape, dtype, layout, nan=False):
+    M, K, N = shape
+    g = torch.Generator().manual_seed(M * 7 + K * 3 + N)
+    W = (torch.randn(K, N, generator=g) / K ** 0.5).to(dtype).cuda()
+    if layout == "features":
+        pass
+    elif layout == "d_in":  # rows padded to 16 B, as an aligned transposed view has them
+        back = torch.zeros(N, -(-K // 8) * 8, dtype=dtype, device="cuda")
+        back[:, :K] = W.T
+        W = back.T[:K]
+    elif layout == "odd_features":  # rows of odd length
+        back = torch.zeros(K, N | 1, dtype=dtype, device="cuda")
+        back[:, :N] = W
+        W = back[:, :N]
+    else:
+        back = torch.zeros(N, K | 1, dtype=dtype, device="cuda")
+        back[:, :K] = W.T
+        W = back[:, :K].T
+    x = torch.randn(M, K, generator=g)
+    if nan:
+        x[M // 2] = float("nan")
+    cut = torch.rand(N, generator=g) * 0.5
+    vec = dict(b_enc=torch.randn(N, generator=g) * 0.1, b_dec=torch.randn(K, generator=g) * 0.1)
+    return x.to(dtype).cuda(), W, {k: v.to(dtype).cuda() for k, v in vec.items()}, cut.to(dtype).cuda()
+
+
+def aligned(shape, dtype, layout):
+    """Whether this W takes the DMA paths (the rows of the 256-feature tiles are not staged otherwise)."""
+    M, K, N = shape
+    if layout == "features":
+        return N % (4 if dtype == torch.float32 else 8) == 0
+    return layout == "d_in" and (K % 2 == 0 or dtype == torch.float32)
+
+
+def same(a, b):
+    bits = {4: torch.int32, 2: torch.int16}[a.element_size()]
+    return torch.equal(a.view(bits), b.view(bits))
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("layout", ["features", "d_in", "odd_features", "odd_d_in"])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_small_tiles_equal_the_wide_tile(dtype, layout, tile):
+    for shape in SHAPES:
+        if tile[1] == 256 and not aligned(shape, dtype, layout):
+            x, W, p, _ = make(shape, dtype, layout)
+            with pytest.raises(ValueError, match="16-B aligned rows"):
+                fused_encode(x, W, p["b_enc"], p["b_dec"], config=config(tile, dtype))
+            continue
+        x, W, p, cut = make(shape, dtype, layout, nan=shape[0] > 100)
+        M = shape[0]
+        for act, out_dtype in (("jumprelu", None), ("relu", torch.float32)):
+            counts = [torch.zeros(M, dtype=torch.int32, device="cuda") for _ in range(2)]
+            got, want = (fused_encode(x, W, p["b_enc"], p["b_dec"], cut, act, out_dtype=out_dtype, row_nnz=n, config=c)
+                         for n, c in zip(counts, (config(tile, dtype), wide(dtype))))
+            assert same(got, want), (shape, act)
+            assert torch.equal(*counts), (shape, act)
+        got, want = (encode_pre(x, W, p["b_enc"], p["b_dec"], config=c) for c in (config(tile, dtype), wide(dtype)))
+        assert same(got, want), shape
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("layout", ["features", "odd_features"])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_small_tile_row_candidates_equal_the_wide_tiles(dtype, layout, tile):
+    for shape in SHAPES:
+        if tile[1] == 256 and not aligned(shape, dtype, layout):
+            continue
+        x, W, p, cut = make(shape, dtype, layout, nan=shape[0] > 100)
+        for act, floor in (("jumprelu", None), ("relu", torch.rand(shape[0], device="cuda")),
+                           ("relu", torch.full((shape[0],), -1.0, device="cuda"))):
+            cap = shape[2] // 3 if floor is None else shape[2]  # some lists overflow
+            lists = []
+            for c in (config(tile, dtype), wide(dtype)):
+                cnt, idx, val = encode_rows(x, W, p["b_enc"], p["b_dec"], cut, act, cap=cap, row_floor=floor, config=c)
+                col = torch.arange(cap, device="cuda")[None]
+                dead = col >= cnt[:, None]
+                order = idx.masked_fill(dead, 1 << 30).sort(dim=1).indices
+                bits = val.view({4: torch.int32, 2: torch.int16}[val.element_size()]).to(torch.int64).masked_fill(dead, 0)
+                lists.append((cnt, idx.masked_fill(dead, 0).gather(1, order), bits.gather(1, order), cnt > cap))
+            (c0, i0, b0, o0), (c1, i1, b1, _) = lists
+            assert torch.equal(c0, c1), (shape, act)
+            ok = ~o0[:, None]  # an overflowed list holds any cap of the kept values
+            assert torch.equal(i0 * ok, i1 * ok) and torch.equal(b0 * ok, b1 * ok), (shape, act)
+
+
+def test_small_tiles_refuse_a_doubly_strided_weight():
+    x, W, p, _ = make((40, 64, 128), torch.bfloat16, "features")
+    W = W.repeat_interleave(2, 0).repeat_interleave(2, 1)[::2, ::2]
+    with pytest.raises(ValueError, match="contiguous along one axis"):
+        fused_encode(x, W, p["b_enc"], p["b_dec"], config=config(TILES[0], torch.bfloat16))
+    assert same(fused_encode(x, W, p["b_enc"], p["b_dec"]), fused_encode(x, W.contiguous(), p["b_enc"], p["b_dec"]))
+
+
+def test_small_tiles_write_a_strided_output_row_in_place():
+    """Output rows that are no 16-B multiple take the element stores: the padding stays as it was."""
+    from saeflow_amd import _lib
+    lib = _lib.load()
+    M, K, N = 70, 96, 203
+    x, W, p, _ = make((M, K, N), torch.bfloat16, "odd_features")
+    want = fused_encode(x, W, p["b_enc"], p["b_dec"], config=wide(torch.bfloat16))
+    out = torch.full((M, N + 6), 7.0, dtype=torch.bfloat16, device="cuda")
+    ws = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+    _lib.check(lib.sf_encode(_lib.ptr(x), K, 1, 1, _lib.ptr(W), W.stride(0), 1, 1, _lib.ptr(p["b_enc"]), 1,
+                             _lib.ptr(p["b_dec"]), 1, None, 0, _lib.ptr(out), N + 6, 1, 1, None, M, N, K, 0, None,
+                             _lib.ptr(ws), ws.numel(), _lib.stream(x.device)))
+    assert same(out[:, :N].contiguous(), want) and bool((out[:, N:] == 7.0).all())
