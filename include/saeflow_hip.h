@@ -147,6 +147,17 @@ SF_API int sf_encode_rows(const void* x, int64_t sxm, int64_t sxk, int x_dt,
                    int64_t M, int64_t N, int64_t K, int act, const int32_t* tile_cfg,
                    void* workspace, int64_t workspace_bytes, void* stream);
 
+/* sf_encode_rows with cand_cnt cleared by the call (in the prologue launch) rather than by the caller;
+ * N > 0. Arguments and results as sf_encode_rows. No reference counterpart (encode.py:130 zeroes its
+ * counter buffer in a launch of its own). */
+SF_API int sf_encode_rows_cleared(const void* x, int64_t sxm, int64_t sxk, int x_dt,
+                   const void* w, int64_t swk, int64_t swn, int w_dt,
+                   const void* b_enc, int benc_dt, const void* b_dec, int bdec_dt,
+                   const void* thr, int thr_dt, const float* row_floor,
+                   int32_t* cand_cnt, int32_t* cand_idx, void* cand_val, int val_dt, int64_t cap,
+                   int64_t M, int64_t N, int64_t K, int act, const int32_t* tile_cfg,
+                   void* workspace, int64_t workspace_bytes, void* stream);
+
 /* The rows whose candidate list overflowed: rows[0 .. n) (int32 [M]) = the m with
  * cand_cnt[m] > cap in increasing order, and *n_rows (int32, device memory) = n, written on
  * the stream, so the caller need not read the counts back. Feeds sf_encode_gather and
@@ -185,6 +196,12 @@ SF_API int sf_rows_to_csr(const int32_t* cand_cnt, const int32_t* cand_idx, cons
                    int64_t cap, int64_t M, const int64_t* indptr, int64_t nnz, int32_t* indices,
                    void* values, void* stream);
 
+/* sf_rows_to_csr for a caller that knows the longest list: with longest at or above every cand_cnt[m],
+ * the launch for lists above 256 entries is left out where there are none. */
+SF_API int sf_rows_to_csr_bounded(const int32_t* cand_cnt, const int32_t* cand_idx, const void* cand_val, int val_dt,
+                   int64_t cap, int64_t M, const int64_t* indptr, int64_t nnz, int64_t longest, int32_t* indices,
+                   void* values, void* stream);
+
 /* Row-wise top-k of row candidates: values [M, k] (val_dt) sorted descending, indices int32
  * [M, k], equal values by increasing column, as sf_topk. A row with fewer than k candidates
  * is completed with zeros at its lowest columns that are not candidates, which equals
@@ -203,6 +220,10 @@ SF_API int sf_count_nonzero(const void* f, int64_t sfm, int64_t sfn, int f_dt,
 /* indptr[0] = 0, indptr[m+1] = sum_{i<=m} counts[i] (int64). Replaces
  * `indptr[1:] = row_nnz.cumsum(0)` (reference decode.py:86-87). */
 SF_API int sf_scan_counts(const int32_t* counts, int64_t M, int64_t* indptr, void* stream);
+
+/* sf_scan_counts that also writes stats[0] = indptr[M] and stats[1] = the largest count (saturated at
+ * 2^20 - 1; 0 if M is 0), both int64 on the device, for the caller's one read back (decode.py:88). */
+SF_API int sf_scan_counts_stats(const int32_t* counts, int64_t M, int64_t* indptr, int64_t* stats, void* stream);
 
 /* Compaction: for every row m, the nonzero elements of f row m, in increasing column
  * order, go to indices/values[indptr[m] ...] (canonical CSR, values copied bit-exact).

@@ -33,13 +33,17 @@ SIGNATURES = {
     "sf_encode_config": (_I32, [_I64, _I64, _I64, _I32, _P]),
     "sf_encode_rows": (_I32, [_P, _I64, _I64, _I32, _P, _I64, _I64, _I32, _P, _I32, _P, _I32, _P, _I32, _P,
                               _P, _P, _P, _I32, _I64, _I64, _I64, _I64, _I32, _P, _P, _I64, _P]),
+    "sf_encode_rows_cleared": (_I32, [_P, _I64, _I64, _I32, _P, _I64, _I64, _I32, _P, _I32, _P, _I32, _P, _I32, _P,
+                                      _P, _P, _P, _I32, _I64, _I64, _I64, _I64, _I32, _P, _P, _I64, _P]),
     "sf_overflow_rows": (_I32, [_P, _I64, _I64, _P, _P, _P]),
     "sf_encode_gather": (_I32, [_P, _I64, _I64, _I32, _I64, _P, _P, _I64, _P, _I64, _I64, _I32, _P, _I32, _P, _I32,
                                 _P, _I32, _P, _I64, _I64, _I32, _I64, _I64, _I64, _I32, _P, _I64, _P]),
     "sf_rows_to_csr": (_I32, [_P, _P, _P, _I32, _I64, _I64, _P, _I64, _P, _P, _P]),
+    "sf_rows_to_csr_bounded": (_I32, [_P, _P, _P, _I32, _I64, _I64, _P, _I64, _I64, _P, _P, _P]),
     "sf_rows_topk": (_I32, [_P, _P, _P, _I32, _I64, _I64, _I64, _I64, _P, _P, _P]),
     "sf_count_nonzero": (_I32, [_P, _I64, _I64, _I32, _I64, _I64, _P, _P]),
     "sf_scan_counts": (_I32, [_P, _I64, _P, _P]),
+    "sf_scan_counts_stats": (_I32, [_P, _I64, _P, _P, _P]),
     "sf_compact": (_I32, [_P, _I64, _I64, _I32, _I64, _I64, _P, _I64, _P, _P, _P]),
     "sf_decode": (_I32, [_P, _P, _P, _I32, _I64, _P, _I64, _I64, _I32, _I64, _P, _I32, _P, _I64, _I64,
                          _I32, _I64, _I64, _P, _P]),

@@ -121,8 +121,15 @@ __global__ __launch_bounds__(256) void count_kernel(const char* f, int64_t sfm, 
 //  2. scan_totals_kernel: one block turns the parked totals into exclusive tile offsets, in
 //     place;
 //  3. scan_final_kernel: each tile reads its offset, then writes its inclusive prefixes.
-// One tile needs only the last pass (offset 0).
+// Up to SCAN_ONE counts take one pass of one block instead (scan_one_kernel): the three launches are
+// 13 us whatever M is, one block's rounds of 16384 counts about 5 us each.
 constexpr int SCAN_PER = 16, SCAN_TILE = 256 * SCAN_PER;
+constexpr int SCAN_ONE_NT = 1024;
+constexpr int64_t SCAN_ONE = 2 * SCAN_ONE_NT * SCAN_PER;
+// Statistics a scan can leave beside indptr: {sum, largest count}. The largest count is carried next
+// to a tile's total (below 2^43: 4096 int32 counts) in one parked word, so it saturates at 2^20 - 1.
+constexpr int STAT_SHIFT = 43;
+constexpr int32_t STAT_MAX = (1 << 20) - 1;
 
 __device__ __forceinline__ void load_counts16(const int32_t* counts, int64_t M, int64_t i0, int32_t (&c)[SCAN_PER]) {
   if (i0 + SCAN_PER <= M && ((uintptr_t)(counts + i0) % 16) == 0) {
@@ -140,39 +147,129 @@ __device__ __forceinline__ void load_counts16(const int32_t* counts, int64_t M, 
   }
 }
 
-__global__ __launch_bounds__(256) void scan_tiles_kernel(const int32_t* counts, int64_t M, int64_t* indptr) {
+__device__ __forceinline__ int32_t wave_max(int32_t v) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) v = max(v, __shfl_xor(v, off));
+  return v;
+}
+
+__global__ __launch_bounds__(256) void scan_tiles_kernel(const int32_t* counts, int64_t M, int64_t* indptr,
+                                                         const int64_t* stats) {
   __shared__ int64_t s_w[4];
+  __shared__ int32_t s_m[4];
   const int64_t i0 = (int64_t)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_PER;
   int32_t c[SCAN_PER];
   load_counts16(counts, M, i0, c);
   int64_t s = 0;
+  int32_t mx = 0;
 #pragma unroll
-  for (int q = 0; q < SCAN_PER; ++q) s += c[q];
+  for (int q = 0; q < SCAN_PER; ++q) {
+    s += c[q];
+    mx = max(mx, c[q]);
+  }
+  if (stats) {
+    mx = wave_max(mx);
+    if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = mx;
+  }
   int64_t total;
-  block_exclusive_i64(s, s_w, total);
-  if (threadIdx.x == 0) indptr[(int64_t)blockIdx.x * SCAN_TILE + 1] = total;
+  block_exclusive_i64(s, s_w, total);  // its barrier orders s_m
+  if (threadIdx.x == 0) {
+    if (stats) {
+      mx = min(max(max(s_m[0], s_m[1]), max(s_m[2], s_m[3])), STAT_MAX);
+      total |= (int64_t)mx << STAT_SHIFT;
+    }
+    indptr[(int64_t)blockIdx.x * SCAN_TILE + 1] = total;
+  }
 }
 
-__global__ __launch_bounds__(256) void scan_totals_kernel(int64_t ntiles, int64_t* indptr) {
+__global__ __launch_bounds__(256) void scan_totals_kernel(int64_t ntiles, int64_t* indptr, int64_t* stats) {
   __shared__ int64_t s_w[4];
+  __shared__ int32_t s_m[4];
   int64_t carry = 0;
+  int32_t mx = 0;
   for (int64_t b0 = 0; b0 < ntiles; b0 += 256) {
     const int64_t b = b0 + threadIdx.x;
-    const int64_t v = b < ntiles ? indptr[b * SCAN_TILE + 1] : 0;
+    int64_t v = b < ntiles ? indptr[b * SCAN_TILE + 1] : 0;
+    if (stats) {
+      mx = max(mx, (int32_t)(v >> STAT_SHIFT));
+      v &= (1ll << STAT_SHIFT) - 1;
+    }
     int64_t total;
     const int64_t ex = block_exclusive_i64(v, s_w, total);
     if (b < ntiles) indptr[b * SCAN_TILE + 1] = carry + ex;
     carry += total;
     __syncthreads();  // s_w is rewritten by the next round
   }
+  if (stats) {
+    mx = wave_max(mx);
+    if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      stats[0] = carry;
+      stats[1] = max(max(s_m[0], s_m[1]), max(s_m[2], s_m[3]));
+    }
+  }
 }
 
-__global__ __launch_bounds__(256) void scan_final_kernel(const int32_t* counts, int64_t M, int64_t* indptr,
-                                                         int has_offsets) {
+// The whole scan by one block of NW waves: rounds of NW x 64 x 16 counts with a running sum.
+template <int NW>
+__global__ __launch_bounds__(NW * 64) void scan_one_kernel(const int32_t* counts, int64_t M, int64_t* indptr,
+                                                           int64_t* stats) {
+  __shared__ int64_t s_w[2][NW];
+  __shared__ int32_t s_m[NW];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  int64_t carry = 0;
+  int32_t mx = 0;
+  int par = 0;
+  for (int64_t r0 = 0; r0 < M; r0 += NW * 64 * SCAN_PER, par ^= 1) {
+    const int64_t i0 = r0 + t * SCAN_PER;
+    int32_t c[SCAN_PER];
+    load_counts16(counts, M, i0, c);
+    int64_t s = 0;
+#pragma unroll
+    for (int q = 0; q < SCAN_PER; ++q) {
+      s += c[q];
+      mx = max(mx, c[q]);
+    }
+    int64_t x = s;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int64_t y = __shfl_up(x, off);
+      if (lane >= off) x += y;
+    }
+    if (lane == 63) s_w[par][w] = x;
+    __syncthreads();  // s_w[par] was last read before the previous round's barrier
+    int64_t run = carry + x - s;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {
+      const int64_t v = s_w[par][q];
+      run += q < w ? v : 0;
+      carry += v;
+    }
+#pragma unroll
+    for (int q = 0; q < SCAN_PER; ++q) {
+      run += c[q];
+      if (i0 + q < M) indptr[i0 + q + 1] = run;
+    }
+  }
+  if (t == 0) indptr[0] = 0;
+  if (stats) {
+    mx = wave_max(mx);
+    if (lane == 0) s_m[w] = mx;
+    __syncthreads();
+    if (t == 0) {
+      for (int q = 1; q < NW; ++q) mx = max(mx, s_m[q]);
+      stats[0] = carry;
+      stats[1] = min(mx, STAT_MAX);
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void scan_final_kernel(const int32_t* counts, int64_t M, int64_t* indptr) {
   __shared__ int64_t s_w[4];
   __shared__ int64_t s_off;
   const int64_t i0 = (int64_t)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_PER;
-  if (threadIdx.x == 0) s_off = has_offsets ? indptr[(int64_t)blockIdx.x * SCAN_TILE + 1] : 0;
+  if (threadIdx.x == 0) s_off = indptr[(int64_t)blockIdx.x * SCAN_TILE + 1];
   int32_t c[SCAN_PER];
   load_counts16(counts, M, i0, c);
   int64_t s = 0;
@@ -599,28 +696,44 @@ __global__ __launch_bounds__(256) void rows_to_csr_kernel(const int32_t* cnt, co
 
 }  // namespace
 
-extern "C" int sf_rows_to_csr(const int32_t* cand_cnt, const int32_t* cand_idx, const void* cand_val, int val_dt,
-                              int64_t cap, int64_t M, const int64_t* indptr, int64_t nnz, int32_t* indices,
-                              void* values, void* stream) {
-  sf_clear_error();
-  SF_REQUIRE(M >= 0 && nnz >= 0, "sf_rows_to_csr: negative size");
-  SF_REQUIRE(sf_valid_dtype(val_dt), "sf_rows_to_csr: bad dtype code %d", val_dt);
-  SF_REQUIRE(cap >= 0 && cap <= SF_ROWS_CAP_MAX, "sf_rows_to_csr: capacity %lld above %d", (long long)cap,
-             SF_ROWS_CAP_MAX);
-  SF_REQUIRE(M < (1LL << 31), "sf_rows_to_csr: too many rows");
+namespace {
+int rows_to_csr_impl(const char* fn, const int32_t* cand_cnt, const int32_t* cand_idx, const void* cand_val, int val_dt,
+                     int64_t cap, int64_t M, const int64_t* indptr, int64_t nnz, int64_t longest, int32_t* indices,
+                     void* values, void* stream) {
+  SF_REQUIRE(M >= 0 && nnz >= 0, "%s: negative size", fn);
+  SF_REQUIRE(sf_valid_dtype(val_dt), "%s: bad dtype code %d", fn, val_dt);
+  SF_REQUIRE(cap >= 0 && cap <= SF_ROWS_CAP_MAX, "%s: capacity %lld above %d", fn, (long long)cap, SF_ROWS_CAP_MAX);
+  SF_REQUIRE(M < (1LL << 31), "%s: too many rows", fn);
   if (M == 0 || nnz == 0 || cap == 0) return SF_OK;
-  SF_REQUIRE(cand_cnt && cand_idx && cand_val && indptr && indices && values, "sf_rows_to_csr: NULL buffer");
+  SF_REQUIRE(cand_cnt && cand_idx && cand_val && indptr && indices && values, "%s: NULL buffer", fn);
   hipLaunchKernelGGL(rows_to_csr_wave_kernel, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
                      cand_cnt, cand_idx, (const char*)cand_val, sf_dtype_size(val_dt), cap, M, indptr, nnz, indices,
                      (char*)values);
   SF_LAUNCH_CHECK("rows_to_csr_wave_kernel");
-  if (cap > WS_MAX) {  // rows longer than the wavefront sort takes
+  if (cap > WS_MAX && longest > WS_MAX) {  // rows longer than the wavefront sort takes
     hipLaunchKernelGGL(rows_to_csr_kernel, dim3((unsigned)((M + LS_ROWS - 1) / LS_ROWS)), dim3(256), 0,
                        (hipStream_t)stream, cand_cnt, cand_idx, (const char*)cand_val, sf_dtype_size(val_dt), cap, M,
                        indptr, nnz, indices, (char*)values);
     SF_LAUNCH_CHECK("rows_to_csr_kernel");
   }
   return SF_OK;
+}
+}  // namespace
+
+extern "C" int sf_rows_to_csr(const int32_t* cand_cnt, const int32_t* cand_idx, const void* cand_val, int val_dt,
+                              int64_t cap, int64_t M, const int64_t* indptr, int64_t nnz, int32_t* indices,
+                              void* values, void* stream) {
+  sf_clear_error();
+  return rows_to_csr_impl("sf_rows_to_csr", cand_cnt, cand_idx, cand_val, val_dt, cap, M, indptr, nnz, INT64_MAX,
+                          indices, values, stream);
+}
+
+extern "C" int sf_rows_to_csr_bounded(const int32_t* cand_cnt, const int32_t* cand_idx, const void* cand_val,
+                                      int val_dt, int64_t cap, int64_t M, const int64_t* indptr, int64_t nnz,
+                                      int64_t longest, int32_t* indices, void* values, void* stream) {
+  sf_clear_error();
+  return rows_to_csr_impl("sf_rows_to_csr_bounded", cand_cnt, cand_idx, cand_val, val_dt, cap, M, indptr, nnz, longest,
+                          indices, values, stream);
 }
 
 extern "C" int sf_count_nonzero(const void* f, int64_t sfm, int64_t sfn, int f_dt, int64_t M, int64_t N,
@@ -648,25 +761,39 @@ extern "C" int sf_count_nonzero(const void* f, int64_t sfm, int64_t sfn, int f_d
   return SF_OK;
 }
 
-extern "C" int sf_scan_counts(const int32_t* counts, int64_t M, int64_t* indptr, void* stream) {
-  sf_clear_error();
-  SF_REQUIRE(M >= 0, "sf_scan_counts: negative size");
-  SF_REQUIRE(indptr && (counts || M == 0), "sf_scan_counts: NULL buffer");
+namespace {
+int scan_impl(const char* fn, const int32_t* counts, int64_t M, int64_t* indptr, int64_t* stats, void* stream) {
+  SF_REQUIRE(M >= 0, "%s: negative size", fn);
+  SF_REQUIRE(indptr && (counts || M == 0), "%s: NULL buffer", fn);
   hipStream_t s = (hipStream_t)stream;
   const int64_t ntiles = (M + SCAN_TILE - 1) / SCAN_TILE;
-  SF_REQUIRE(ntiles < (1LL << 31), "sf_scan_counts: too many counts");
-  if (ntiles <= 1) {
-    hipLaunchKernelGGL(scan_final_kernel, dim3(1), dim3(256), 0, s, counts, M, indptr, 0);
-    SF_LAUNCH_CHECK("scan_final_kernel");
+  SF_REQUIRE(ntiles < (1LL << 31), "%s: too many counts", fn);
+  if (M <= SCAN_ONE) {
+    const unsigned nt = M <= 4 * 64 * SCAN_PER ? 256 : SCAN_ONE_NT;
+    if (nt == 256) hipLaunchKernelGGL(scan_one_kernel<4>, dim3(1), dim3(256), 0, s, counts, M, indptr, stats);
+    else hipLaunchKernelGGL(scan_one_kernel<SCAN_ONE_NT / 64>, dim3(1), dim3(SCAN_ONE_NT), 0, s, counts, M, indptr, stats);
+    SF_LAUNCH_CHECK("scan_one_kernel");
     return SF_OK;
   }
-  hipLaunchKernelGGL(scan_tiles_kernel, dim3((unsigned)ntiles), dim3(256), 0, s, counts, M, indptr);
+  hipLaunchKernelGGL(scan_tiles_kernel, dim3((unsigned)ntiles), dim3(256), 0, s, counts, M, indptr, stats);
   SF_LAUNCH_CHECK("scan_tiles_kernel");
-  hipLaunchKernelGGL(scan_totals_kernel, dim3(1), dim3(256), 0, s, ntiles, indptr);
+  hipLaunchKernelGGL(scan_totals_kernel, dim3(1), dim3(256), 0, s, ntiles, indptr, stats);
   SF_LAUNCH_CHECK("scan_totals_kernel");
-  hipLaunchKernelGGL(scan_final_kernel, dim3((unsigned)ntiles), dim3(256), 0, s, counts, M, indptr, 1);
+  hipLaunchKernelGGL(scan_final_kernel, dim3((unsigned)ntiles), dim3(256), 0, s, counts, M, indptr);
   SF_LAUNCH_CHECK("scan_final_kernel");
   return SF_OK;
+}
+}  // namespace
+
+extern "C" int sf_scan_counts(const int32_t* counts, int64_t M, int64_t* indptr, void* stream) {
+  sf_clear_error();
+  return scan_impl("sf_scan_counts", counts, M, indptr, nullptr, stream);
+}
+
+extern "C" int sf_scan_counts_stats(const int32_t* counts, int64_t M, int64_t* indptr, int64_t* stats, void* stream) {
+  sf_clear_error();
+  SF_REQUIRE(stats, "sf_scan_counts_stats: NULL buffer");
+  return scan_impl("sf_scan_counts_stats", counts, M, indptr, stats, stream);
 }
 
 extern "C" int sf_compact(const void* f, int64_t sfm, int64_t sfn, int f_dt, int64_t M, int64_t N,

@@ -27,7 +27,8 @@ hipError_t launch_xprep_rows(const void* x, int64_t sxm, int64_t sxk, int x_dt, 
 
 template <int DT>
 hipError_t launch_xprep(const void* x, int64_t sxm, int64_t sxk, int x_dt, const void* b_dec, int bdec_dt,
-                        int64_t M, int64_t K, int64_t Kp, char* xw, int32_t* tile_ctr, hipStream_t s) {
+                        int64_t M, int64_t K, int64_t Kp, char* xw, int32_t* tile_ctr, int32_t* clear,
+                        hipStream_t s) {
   constexpr int E = Traits<DT>::E, EPC = Traits<DT>::EPC;
   const bool fast = x_dt == DT && bdec_dt == DT && sxk == 1 && (K % EPC) == 0 && ((uintptr_t)x % 16) == 0 &&
                     ((sxm * E) % 16) == 0 && ((uintptr_t)b_dec % 16) == 0;
@@ -35,10 +36,10 @@ hipError_t launch_xprep(const void* x, int64_t sxm, int64_t sxk, int x_dt, const
   const unsigned blocks = (unsigned)std::min<int64_t>((chunks + 255) / 256, 65536);
   if (fast)
     hipLaunchKernelGGL((xprep_kernel<DT, true>), dim3(blocks), dim3(256), 0, s, x, sxm, sxk, x_dt, b_dec, bdec_dt,
-                       M, K, Kp, xw, tile_ctr);
+                       M, K, Kp, xw, tile_ctr, clear);
   else
     hipLaunchKernelGGL((xprep_kernel<DT, false>), dim3(blocks), dim3(256), 0, s, x, sxm, sxk, x_dt, b_dec, bdec_dt,
-                       M, K, Kp, xw, tile_ctr);
+                       M, K, Kp, xw, tile_ctr, clear);
   return hipGetLastError();
 }
 
@@ -185,7 +186,7 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
                 int32_t* cand_cnt, int32_t* cand_idx, void* cand_val, int64_t cap, const float* row_floor,
                 int64_t M, int64_t N, int64_t K, int act, const int32_t* tile_cfg, void* workspace,
                 int64_t workspace_bytes, void* stream, bool gather = false, const int32_t* live_rows = nullptr,
-                const int32_t* n_live = nullptr, int64_t live_off = 0, int64_t Mx = 0) {
+                const int32_t* n_live = nullptr, int64_t live_off = 0, int64_t Mx = 0, bool clear_cnt = false) {
   SF_REQUIRE(M >= 0 && N >= 0 && K >= 0, "%s: negative size (M=%lld N=%lld K=%lld)", fn, (long long)M,
              (long long)N, (long long)K);
   SF_REQUIRE(sf_valid_dtype(x_dt) && sf_valid_dtype(w_dt) && sf_valid_dtype(benc_dt) &&
@@ -323,10 +324,11 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
     if (e != hipSuccess) return sf_fail(SF_EHIP, "%s: kernel launch failed: %s", fn, hipGetErrorString(e));
     return SF_OK;
   }
+  int32_t* const clear = clear_cnt ? cand_cnt : nullptr;
   switch (w_dt) {
-    case SF_BF16: e = launch_xprep<SF_BF16>(x, sxm, sxk, x_dt, b_dec, bdec_dt, M, K, Kp, (char*)workspace, a.tile_ctr, s); break;
-    case SF_F16: e = launch_xprep<SF_F16>(x, sxm, sxk, x_dt, b_dec, bdec_dt, M, K, Kp, (char*)workspace, a.tile_ctr, s); break;
-    default: e = launch_xprep<SF_F32>(x, sxm, sxk, x_dt, b_dec, bdec_dt, M, K, Kp, (char*)workspace, a.tile_ctr, s); break;
+    case SF_BF16: e = launch_xprep<SF_BF16>(x, sxm, sxk, x_dt, b_dec, bdec_dt, M, K, Kp, (char*)workspace, a.tile_ctr, clear, s); break;
+    case SF_F16: e = launch_xprep<SF_F16>(x, sxm, sxk, x_dt, b_dec, bdec_dt, M, K, Kp, (char*)workspace, a.tile_ctr, clear, s); break;
+    default: e = launch_xprep<SF_F32>(x, sxm, sxk, x_dt, b_dec, bdec_dt, M, K, Kp, (char*)workspace, a.tile_ctr, clear, s); break;
   }
   if (e != hipSuccess) return sf_fail(SF_EHIP, "%s: prologue launch failed: %s", fn, hipGetErrorString(e));
   if (slim >= 0) {
@@ -373,6 +375,20 @@ extern "C" int sf_encode_rows(const void* x, int64_t sxm, int64_t sxk, int x_dt,
                      cand_val, cap, row_floor, M, N, K, act, tile_cfg, workspace, workspace_bytes, stream);
 }
 
+
+extern "C" int sf_encode_rows_cleared(const void* x, int64_t sxm, int64_t sxk, int x_dt, const void* w, int64_t swk,
+                                      int64_t swn, int w_dt, const void* b_enc, int benc_dt, const void* b_dec,
+                                      int bdec_dt, const void* thr, int thr_dt, const float* row_floor,
+                                      int32_t* cand_cnt, int32_t* cand_idx, void* cand_val, int val_dt, int64_t cap,
+                                      int64_t M, int64_t N, int64_t K, int act, const int32_t* tile_cfg,
+                                      void* workspace, int64_t workspace_bytes, void* stream) {
+  sf_clear_error();
+  SF_REQUIRE(N > 0 || M <= 0, "sf_encode_rows_cleared: no features, so no launch to clear the counts in");
+  return encode_impl("sf_encode_rows_cleared", row_floor ? EPI_ROWS_FLOOR : EPI_ROWS, x, sxm, sxk, x_dt, w, swk, swn,
+                     w_dt, b_enc, benc_dt, b_dec, bdec_dt, thr, thr_dt, nullptr, 0, 0, val_dt, nullptr, cand_cnt,
+                     cand_idx, cand_val, cap, row_floor, M, N, K, act, tile_cfg, workspace, workspace_bytes, stream,
+                     false, nullptr, nullptr, 0, 0, true);
+}
 
 extern "C" int sf_encode_gather(const void* x, int64_t sxm, int64_t sxk, int x_dt, int64_t Mx, const int32_t* rows,
                                 const int32_t* n_rows, int64_t row_off, const void* w, int64_t swk, int64_t swn,

@@ -203,8 +203,11 @@ __device__ __forceinline__ u32x4 pack_chunk(const float* v) {
 template <int DT, bool FAST>
 __global__ __launch_bounds__(256) void xprep_kernel(const void* x, int64_t sxm, int64_t sxk, int x_dt,
                                                     const void* b_dec, int bdec_dt, int64_t M, int64_t K,
-                                                    int64_t Kp, char* xw, int32_t* tile_ctr) {
+                                                    int64_t Kp, char* xw, int32_t* tile_ctr, int32_t* clear) {
   constexpr int E = Traits<DT>::E, EPC = Traits<DT>::EPC;
+  // the row-candidate GEMM that follows counts from zero (clear: its counts [M], or NULL)
+  if (clear)
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < M; i += (int64_t)gridDim.x * 256) clear[i] = 0;
   // the GEMM that follows on the stream claims tiles from these (persistent form)
   if (blockIdx.x == 0 && threadIdx.x < 8) tile_ctr[threadIdx.x * TILE_CTR_STRIDE] = 0;
   const int64_t cpr = Kp / EPC;  // chunks per row

@@ -37,6 +37,21 @@ def exclusive_scan(row_nnz):
     return indptr
 
 
+def scan_counts(row_nnz):
+    """(indptr, nnz, longest): exclusive_scan(row_nnz) and, read back with one host synchronisation,
+    its last entry and the largest count (at most 2^20 - 1 is reported)."""
+    M = row_nnz.numel()
+    dev = _lib.require_gpu(("row_nnz", row_nnz))
+    row_nnz = row_nnz.reshape(M).to(torch.int32).contiguous()
+    indptr = torch.empty(M + 1, dtype=torch.int64, device=row_nnz.device)
+    stats = torch.empty(2, dtype=torch.int64, device=row_nnz.device)
+    with torch.cuda.device(dev):
+        _lib.check(_lib.load().sf_scan_counts_stats(_lib.ptr(row_nnz), M, _lib.ptr(indptr), _lib.ptr(stats),
+                                                    _lib.stream(dev)))
+    nnz, longest = stats.tolist()
+    return indptr, nnz, longest
+
+
 def compact(f, indptr, nnz):
     """(indices int32 [nnz], values [nnz]): the nonzeros of every row of f in column order,
     placed at indptr[row] (_compact_kernel, decode.py:61-74)."""
@@ -66,8 +81,7 @@ def dense_to_csr(f, row_nnz=None):
         row_nnz = row_counts(f)
     elif row_nnz.numel() != M:
         raise ValueError(f"row_nnz has {row_nnz.numel()} entries, f has {M} rows")
-    indptr = exclusive_scan(row_nnz)
-    nnz = int(indptr[-1])
+    indptr, nnz, _ = scan_counts(row_nnz)
     indices, values = compact(f, indptr, nnz)
     return indptr, indices, values
 
@@ -215,9 +229,9 @@ def fixed_width_to_dense(indices, values, d_sae):
     return out
 
 
-def rows_to_csr(cand_cnt, cand_idx, cand_val, indptr, nnz):
+def rows_to_csr(cand_cnt, cand_idx, cand_val, indptr, nnz, longest=None):
     """Row candidates (encode_rows) -> canonical CSR (indices int32 [nnz], values [nnz]), rows
-    sorted by column; indptr = exclusive_scan(cand_cnt). Rows whose list overflowed (cand_cnt >
+    sorted by column; indptr = exclusive_scan(cand_cnt); longest: a bound of the counts, if known. Rows whose list overflowed (cand_cnt >
     cap) are skipped: their segments of the returned arrays are left unset for the caller to
     fill (as ops._fill_overflowed_rows does)."""
     M, cap = cand_idx.shape
@@ -229,9 +243,10 @@ def rows_to_csr(cand_cnt, cand_idx, cand_val, indptr, nnz):
         return indices, values
     lib = _lib.load()
     with torch.cuda.device(dev):
-        _lib.check(lib.sf_rows_to_csr(_lib.ptr(cand_cnt), _lib.ptr(cand_idx), _lib.ptr(cand_val),
-                                      _lib.dtype_code(cand_val, "cand_val"), cap, M, _lib.ptr(indptr), nnz,
-                                      _lib.ptr(indices), _lib.ptr(values), _lib.stream(dev)))
+        _lib.check(lib.sf_rows_to_csr_bounded(_lib.ptr(cand_cnt), _lib.ptr(cand_idx), _lib.ptr(cand_val),
+                                              _lib.dtype_code(cand_val, "cand_val"), cap, M, _lib.ptr(indptr), nnz,
+                                              cap if longest is None else longest, _lib.ptr(indices),
+                                              _lib.ptr(values), _lib.stream(dev)))
     return indices, values
 
 

@@ -7,8 +7,8 @@ see kernels/decode.py.
 
 import torch
 
-from .kernels import (dense_to_csr, encode_gather, encode_rows, exclusive_scan, fixed_width_to_dense, fused_encode,
-                      overflow_rows, rows_to_csr, rows_topk, sparse_decode, topk_gather, topk_rows)
+from .kernels import (dense_to_csr, encode_gather, encode_rows, fixed_width_to_dense, fused_encode,
+                      overflow_rows, rows_to_csr, rows_topk, scan_counts, sparse_decode, topk_gather, topk_rows)
 
 # Row-candidate paths: the fused encode appends each row's selected features to a per-row list
 # instead of writing the dense [M, d_sae] features, which the reference writes and reads back
@@ -95,9 +95,8 @@ def _encode_sparse_rows(sae, x):
     counts and its one host read (nnz, as dense_to_csr, decode.py:88) also bring back the
     longest list; rows longer than ROW_CAP are filled in by _fill_overflowed_rows."""
     cnt, idx, val = encode_rows(x, sae.W_enc, sae.b_enc, sae.b_dec, sae.threshold, sae.activation, cap=ROW_CAP)
-    indptr = exclusive_scan(cnt)
-    nnz, longest = torch.stack([indptr[-1], cnt.max().to(torch.int64)]).tolist()
-    indices, values = rows_to_csr(cnt, idx, val, indptr, nnz)  # overflowed rows are skipped
+    indptr, nnz, longest = scan_counts(cnt)
+    indices, values = rows_to_csr(cnt, idx, val, indptr, nnz, longest)  # overflowed rows are skipped
     if longest > ROW_CAP:
         _fill_overflowed_rows(sae, x, cnt, indptr, indices, values)
     return indptr, indices, values

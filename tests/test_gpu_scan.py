@@ -1,0 +1,53 @@
+"""GPU: the count scan that sizes a CSR (one block up to 32768 rows, three passes above), the numbers
+it leaves for the host, and the row-candidate calls that use them."""
+
+import pytest
+import torch
+
+from saeflow_amd.kernels import encode_rows, exclusive_scan, rows_to_csr, scan_counts
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [0, 1, 15, 16, 17, 4095, 4096, 4097, 16384, 16385, 32768, 32769, 300001])
+@pytest.mark.parametrize("offset", [0, 1])  # counts that are 16-B aligned or not
+def test_scan_counts(M, offset):
+    g = torch.Generator().manual_seed(M)
+    counts = torch.randint(0, 1000, (M + offset,), generator=g, dtype=torch.int32)[offset:]
+    if M > 2:
+        counts[M // 2] = 70000  # sums beyond 2^31 at the largest M would not show otherwise
+    dev = torch.cat([torch.zeros(offset, dtype=torch.int32), counts]).cuda()[offset:]
+    indptr, nnz, longest = scan_counts(dev)
+    want = torch.cat([torch.zeros(1, dtype=torch.int64), counts.long().cumsum(0)])
+    assert torch.equal(indptr.cpu(), want) and torch.equal(exclusive_scan(dev).cpu(), want)
+    assert nnz == int(want[-1]) and longest == (int(counts.max()) if M else 0)
+
+
+@pytest.mark.parametrize("M", [3, 40000])
+def test_scan_counts_of_large_counts(M):
+    """Sums past 2^31; a largest count of 2^20 and more is reported as 2^20 - 1."""
+    counts = torch.full((M,), 1 << 20, dtype=torch.int32)
+    counts[-1] = 2 ** 31 - 1
+    indptr, nnz, longest = scan_counts(counts.cuda())
+    assert nnz == (M - 1) * (1 << 20) + 2 ** 31 - 1 == int(indptr[-1]) and longest == (1 << 20) - 1
+    counts[-1] = 5
+    assert scan_counts(counts.cuda())[2] == (1 << 20) - 1
+
+
+@pytest.mark.parametrize("M", [1, 300])
+def test_row_candidates_count_from_zero_and_sort_with_a_known_bound(M):
+    """encode_rows clears its counts whatever the memory held; rows_to_csr with the longest list known
+    equals the call without it, with and without lists above 256 entries."""
+    for b in (-1.0, 1.0):  # few and nearly all of the 600 features kept
+        x = torch.randn(M, 64, generator=torch.Generator().manual_seed(1)).cuda()
+        W = torch.randn(64, 600, generator=torch.Generator().manual_seed(2)).cuda() / 8
+        b_enc = torch.full((600,), b, device="cuda")
+        junk = torch.full((M,), 12345, dtype=torch.int32, device="cuda")
+        del junk  # its block is what the counts are likely to get
+        cnt, idx, val = encode_rows(x, W, b_enc, torch.zeros(64, device="cuda"), cap=1024)
+        f = torch.relu(x.double() @ W.double() + b)
+        assert torch.equal(cnt.cpu(), (f > 0).sum(1).int().cpu())
+        indptr, nnz, longest = scan_counts(cnt)
+        assert (longest > 256) == (b > 0)
+        for a, c in zip(rows_to_csr(cnt, idx, val, indptr, nnz, longest), rows_to_csr(cnt, idx, val, indptr, nnz)):
+            assert torch.equal(a, c)
