@@ -88,15 +88,17 @@ __device__ __forceinline__ void row_range(const DecArgs& a, int64_t row, int64_t
 // Store output chunk d0 .. d0+EPC-1 of `row` (fp32 sums + b_dec, cast to the output type):
 // one 16-B store when the output is row-contiguous, aligned and of W_dec's width, else
 // element by element through the strides.
+// `bias`: the chunk's b_dec values where the caller has loaded them, else NULL.
 template <int ES>
-__device__ __forceinline__ void store_chunk(const DecArgs& a, int64_t row, int64_t d0, const float* acc) {
+__device__ __forceinline__ void store_chunk(const DecArgs& a, int64_t row, int64_t d0, const float* acc,
+                                            const float* bias = nullptr) {
   constexpr int EPC = 16 / ES;
   const int oes = sf_dtype_size(a.out_dt);
   uint32_t bits[EPC];
 #pragma unroll
   for (int e = 0; e < EPC; ++e) {
     float o = acc[e];
-    if (a.b_dec) o += load_as_f32(a.b_dec, a.bdec_dt, d0 + e);
+    if (a.b_dec) o += bias ? bias[e] : load_as_f32(a.b_dec, a.bdec_dt, d0 + e);
     bits[e] = f32_to_bits(o, a.out_dt);
   }
   if (a.vec_out && oes == ES) {
@@ -188,6 +190,13 @@ __global__ __launch_bounds__(256) void decode_vec_kernel(DecArgs a) {
 constexpr int LR_BUF = 4, LU_BUF = 4;
 constexpr int LR_BUF2 = 4, LU_BUF2 = 2;  // two-line slabs: rounds of 2 rows (C3 2-3% faster than 4)
 constexpr int LR_GLB = 10, LU_GLB = 4;
+// At most one workgroup per CU: too few wavefronts to hide a round's latency, so rounds of 16 rows,
+// 32 in flight, and the bias loaded ahead. Measured (us, bf16 d_in 2304, 64 entries a token):
+// d_sae 16384, 1 token 9.6 -> 8.6, 32 tokens 14.3 -> 9.9, 137 tokens 14.8 -> 10.7; d_sae 2^20, 137 tokens
+// 18.6 -> 16.2. From 288 workgroups (256 tokens) on the two are even or the smaller rounds, whose
+// registers leave room for more wavefronts, are faster (d_sae 65536, 512 tokens 23 against 27).
+constexpr int LR_FEW = 4, LR_FEW_GLB = 8, LU_FEW = 16;
+constexpr int64_t LINES_FEW_WG = 256;
 constexpr int LG = 8;   // tokens per wavefront with one-line slabs
 
 struct LineArgs {
@@ -237,6 +246,12 @@ __global__ __launch_bounds__(256) void decode_lines_kernel(LineArgs la) {
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(a.w + slab * 128 * SL), (short)(a.swn * ES), (int)a.d_sae, (int)SF_RSRC_W3);
   const char* wcol = a.w + ch * 16;
+  constexpr bool FEW = LU == LU_FEW;
+  float bias[FEW ? EPC : 1];
+  if constexpr (FEW)
+    if (a.b_dec)
+#pragma unroll
+      for (int e = 0; e < EPC; ++e) bias[e] = load_as_f32(a.b_dec, a.bdec_dt, ch * EPC + e);
   constexpr int NR = B / LU;  // rounds of a batch
 
   for (int64_t j0 = 0; j0 < nmax; j0 += B) {
@@ -307,7 +322,7 @@ __global__ __launch_bounds__(256) void decode_lines_kernel(LineArgs la) {
       }
     }
   }
-  if (tok_on) store_chunk<ES>(a, row, ch * EPC, acc);
+  if (tok_on) store_chunk<ES>(a, row, ch * EPC, acc, FEW ? bias : nullptr);
 }
 
 // generic path: any W_dec strides/alignment, any D. Lane owns elements lane + 64 i of
@@ -391,7 +406,16 @@ hipError_t launch_wdt(const DecArgs& a, bool vec, int nc_cfg, hipStream_t s) {
     if (la.per * 8 <= 0x7fffffffLL) {  // else the grid would not fit: the row kernel below
       const bool buf = a.swn * ES <= 16383 && a.d_sae * a.swn * ES < (1LL << 31);
       const dim3 grid((unsigned)(la.per * 8)), block(256);
-      if (buf && sl == 2)
+      if (la.tot <= LINES_FEW_WG) {
+        if (buf && sl == 2)
+          hipLaunchKernelGGL((decode_lines_kernel<WDT, true, LR_FEW, LU_FEW, 2>), grid, block, 0, s, la);
+        else if (buf)
+          hipLaunchKernelGGL((decode_lines_kernel<WDT, true, LR_FEW, LU_FEW, 1>), grid, block, 0, s, la);
+        else if (sl == 2)
+          hipLaunchKernelGGL((decode_lines_kernel<WDT, false, LR_FEW_GLB, LU_FEW, 2>), grid, block, 0, s, la);
+        else
+          hipLaunchKernelGGL((decode_lines_kernel<WDT, false, LR_FEW_GLB, LU_FEW, 1>), grid, block, 0, s, la);
+      } else if (buf && sl == 2)
         hipLaunchKernelGGL((decode_lines_kernel<WDT, true, LR_BUF2, LU_BUF2, 2>), grid, block, 0, s, la);
       else if (buf)
         hipLaunchKernelGGL((decode_lines_kernel<WDT, true, LR_BUF, LU_BUF, 1>), grid, block, 0, s, la);
