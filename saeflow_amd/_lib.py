@@ -6,7 +6,9 @@ over from torch tensors then belong to the same runtime. There is no fallback: w
 the built library, or with tensors that are not on a ROCm device, every op raises.
 """
 
+import contextlib
 import ctypes
+import functools
 import threading
 from pathlib import Path
 
@@ -123,6 +125,24 @@ def require_gpu(*named):
     return dev
 
 
-def stream(device):
-    """torch's current stream on `device`, as the hipStream_t handle the C ABI takes."""
-    return torch.cuda.current_stream(device).cuda_stream
+_on_device = contextlib.nullcontext()  # stateless, so one object serves every thread
+
+
+def device(dev):
+    """Context in which `dev` is the current device; the usual case, that it already is, costs 0.3 us
+    in place of the device guard's 1.2."""
+    return _on_device if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+
+
+def stream(dev):
+    """torch's current stream on `dev`, as the hipStream_t handle the C ABI takes (0.1 us; building a
+    torch.cuda.Stream object for it costs 1.8)."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
+
+
+@functools.lru_cache(maxsize=256)
+def encode_workspace_bytes(M, K, w_code):
+    """sf_encode_workspace_size, a function of its arguments alone."""
+    nbytes = ctypes.c_int64()
+    check(load().sf_encode_workspace_size(M, K, w_code, ctypes.byref(nbytes)))
+    return nbytes.value

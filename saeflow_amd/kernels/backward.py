@@ -40,7 +40,7 @@ def csr_transpose(indptr, indices, n_cols):
     nbytes = ctypes.c_int64()
     _lib.check(lib.sf_csr_transpose_workspace_size(M, n_cols, nnz, ctypes.byref(nbytes)))
     ws = torch.empty(nbytes.value, dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(lib.sf_csr_transpose(_lib.ptr(indptr), _lib.ptr(indices), M, n_cols, nnz, _lib.ptr(colptr),
                                         _lib.ptr(rows), _lib.ptr(pos), _lib.ptr(ws), nbytes.value,
                                         _lib.stream(dev)))
@@ -73,7 +73,7 @@ def sparse_backward(x, W_enc, b_enc, W_dec, b_dec, csr, grad_x_hat=None, grad_va
     code = _lib.dtype_code(W_dec, "W_dec")
     nnz = indices.numel()
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         s = _lib.stream(dev)
         g = torch.zeros(M, D, dtype=dt, device=dev) if grad_x_hat is None else _rows(grad_x_hat, dt)
         Wd = _rows(W_dec, dt)

@@ -20,7 +20,7 @@ def row_counts(f):
     dev = _lib.require_gpu(("f", f))
     counts = torch.empty(M, dtype=torch.int32, device=f.device)
     if M:
-        with torch.cuda.device(dev):
+        with _lib.device(dev):
             _lib.check(_lib.load().sf_count_nonzero(_lib.ptr(f), f.stride(0), f.stride(1), _lib.dtype_code(f, "f"),
                                                     M, N, _lib.ptr(counts), _lib.stream(dev)))
     return counts
@@ -32,7 +32,7 @@ def exclusive_scan(row_nnz):
     dev = _lib.require_gpu(("row_nnz", row_nnz))
     row_nnz = row_nnz.reshape(M).to(torch.int32).contiguous()
     indptr = torch.empty(M + 1, dtype=torch.int64, device=row_nnz.device)
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(_lib.load().sf_scan_counts(_lib.ptr(row_nnz), M, _lib.ptr(indptr), _lib.stream(dev)))
     return indptr
 
@@ -45,7 +45,7 @@ def scan_counts(row_nnz):
     row_nnz = row_nnz.reshape(M).to(torch.int32).contiguous()
     indptr = torch.empty(M + 1, dtype=torch.int64, device=row_nnz.device)
     stats = torch.empty(2, dtype=torch.int64, device=row_nnz.device)
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(_lib.load().sf_scan_counts_stats(_lib.ptr(row_nnz), M, _lib.ptr(indptr), _lib.ptr(stats),
                                                     _lib.stream(dev)))
     nnz, longest = stats.tolist()
@@ -60,7 +60,7 @@ def compact(f, indptr, nnz):
     indices = torch.empty(nnz, dtype=torch.int32, device=f.device)
     values = torch.empty(nnz, dtype=f.dtype, device=f.device)
     if nnz and M:
-        with torch.cuda.device(dev):
+        with _lib.device(dev):
             _lib.check(_lib.load().sf_compact(_lib.ptr(f), f.stride(0), f.stride(1), _lib.dtype_code(f, "f"), M, N,
                                               _lib.ptr(indptr), nnz, _lib.ptr(indices), _lib.ptr(values),
                                               _lib.stream(dev)))
@@ -131,7 +131,7 @@ def sparse_decode(indptr, indices, values, W_dec, b_dec=None, *, out_dtype=None,
         except (TypeError, KeyError, ValueError):
             raise ValueError(f"config must be a dict with BLOCK_NNZ and BLOCK_D, got {config!r}") from None
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(lib.sf_decode(
             _lib.ptr(indptr), _lib.ptr(indices), _lib.ptr(values), _lib.dtype_code(values, "values"), values.numel(),
             _lib.ptr(W_dec), W_dec.stride(0), W_dec.stride(1), _lib.dtype_code(W_dec, "W_dec"), d_sae,
@@ -150,7 +150,7 @@ def csr_to_dense(indptr, indices, values, d_sae):
     indptr, indices, values = _csr_parts(indptr, indices, values)
     lib = _lib.load()
     code = _lib.dtype_code(values, "values")
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(lib.sf_csr_to_dense(_lib.ptr(indptr), 0, _lib.ptr(indices), _lib.ptr(values), code,
                                        values.numel(), M, d_sae, _lib.ptr(out), out.stride(0), code,
                                        _lib.stream(dev)))
@@ -172,7 +172,7 @@ def topk_rows(f, k):
         return values, indices
     dev = _lib.require_gpu(("f", f))
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(lib.sf_topk(_lib.ptr(f), f.stride(0), f.stride(1), _lib.dtype_code(f, "f"), M, N, k,
                                _lib.ptr(values), _lib.ptr(indices), _lib.stream(dev)))
     return values, indices
@@ -192,7 +192,7 @@ def topk_gather(f, k, n_rows, out_rows, values, indices, *, row_off=0):
         return
     dev = _lib.require_gpu(("f", f), ("n_rows", n_rows), ("out_rows", out_rows), ("values", values),
                            ("indices", indices))
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(_lib.load().sf_topk_gather(_lib.ptr(f), f.stride(0), f.stride(1), _lib.dtype_code(f, "f"), M, N, k,
                                               _lib.ptr(n_rows), row_off, _lib.ptr(out_rows), values.shape[0],
                                               _lib.ptr(values), _lib.ptr(indices), _lib.stream(dev)))
@@ -205,7 +205,7 @@ def overflow_rows(cand_cnt, cap):
     dev = _lib.require_gpu(("cand_cnt", cand_cnt))
     rows = torch.empty(M, dtype=torch.int32, device=cand_cnt.device)
     n = torch.empty(1, dtype=torch.int32, device=cand_cnt.device)
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(_lib.load().sf_overflow_rows(_lib.ptr(cand_cnt.contiguous()), M, cap, _lib.ptr(rows), _lib.ptr(n),
                                                 _lib.stream(dev)))
     return rows, n
@@ -223,7 +223,7 @@ def fixed_width_to_dense(indices, values, d_sae):
     values = values.contiguous()
     lib = _lib.load()
     code = _lib.dtype_code(values, "values")
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(lib.sf_csr_to_dense(None, k, _lib.ptr(indices), _lib.ptr(values), code, values.numel(), M, d_sae,
                                        _lib.ptr(out), out.stride(0), code, _lib.stream(dev)))
     return out
@@ -242,7 +242,7 @@ def rows_to_csr(cand_cnt, cand_idx, cand_val, indptr, nnz, longest=None):
     if M == 0 or nnz == 0:
         return indices, values
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(lib.sf_rows_to_csr_bounded(_lib.ptr(cand_cnt), _lib.ptr(cand_idx), _lib.ptr(cand_val),
                                               _lib.dtype_code(cand_val, "cand_val"), cap, M, _lib.ptr(indptr), nnz,
                                               cap if longest is None else longest, _lib.ptr(indices),
@@ -262,7 +262,7 @@ def rows_topk(cand_cnt, cand_idx, cand_val, k, n_features):
     if M == 0 or k == 0:
         return values, indices
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.device(dev):
         _lib.check(lib.sf_rows_topk(_lib.ptr(cand_cnt), _lib.ptr(cand_idx), _lib.ptr(cand_val),
                                     _lib.dtype_code(cand_val, "cand_val"), cap, M, n_features, k,
                                     _lib.ptr(values), _lib.ptr(indices), _lib.stream(dev)))

@@ -119,14 +119,12 @@ def _launch(x, W_enc, b_enc, b_dec, threshold, act, out, row_nnz, config):
     lib = _lib.load()
     thr_code = _lib.dtype_code(threshold, "threshold") if threshold is not None else 0
     w_code = _lib.dtype_code(W_enc, "W_enc")
-    nbytes = ctypes.c_int64()
-    _lib.check(lib.sf_encode_workspace_size(M, K, w_code, ctypes.byref(nbytes)))
     # x' = cast(x - b_dec) scratch (from torch's caching allocator, reused across calls)
-    ws = torch.empty(max(nbytes.value, 16), dtype=torch.uint8, device=x.device)
+    ws = torch.empty(max(_lib.encode_workspace_bytes(M, K, w_code), 16), dtype=torch.uint8, device=x.device)
 
     def launch(config):
         cfg = _config_array(config, W_enc.dtype)
-        with torch.cuda.device(dev):
+        with _lib.device(dev):
             _lib.check(lib.sf_encode(
                 _lib.ptr(x), x.stride(0), x.stride(1), _lib.dtype_code(x, "x"),
                 _lib.ptr(W_enc), W_enc.stride(0), W_enc.stride(1), w_code,
@@ -243,10 +241,8 @@ def encode_rows(x, W_enc, b_enc, b_dec, threshold=None, activation="relu", *, ca
     cfg = _config_array(config, W_enc.dtype)
     lib = _lib.load()
     w_code = _lib.dtype_code(W_enc, "W_enc")
-    nbytes = ctypes.c_int64()
-    _lib.check(lib.sf_encode_workspace_size(M, K, w_code, ctypes.byref(nbytes)))
-    ws = torch.empty(max(nbytes.value, 16), dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(dev):
+    ws = torch.empty(max(_lib.encode_workspace_bytes(M, K, w_code), 16), dtype=torch.uint8, device=x.device)
+    with _lib.device(dev):
         _lib.check(lib.sf_encode_rows_cleared(
             _lib.ptr(x), x.stride(0), x.stride(1), _lib.dtype_code(x, "x"),
             _lib.ptr(W_enc), W_enc.stride(0), W_enc.stride(1), w_code,
@@ -286,10 +282,8 @@ def encode_gather(x, W_enc, b_enc, b_dec, rows, n_rows, threshold=None, activati
         threshold = _vector(threshold, N, "threshold")
     lib = _lib.load()
     w_code = _lib.dtype_code(W_enc, "W_enc")
-    nbytes = ctypes.c_int64()
-    _lib.check(lib.sf_encode_workspace_size(out_rows, K, w_code, ctypes.byref(nbytes)))
-    ws = torch.empty(max(nbytes.value, 16), dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(dev):
+    ws = torch.empty(max(_lib.encode_workspace_bytes(out_rows, K, w_code), 16), dtype=torch.uint8, device=x.device)
+    with _lib.device(dev):
         _lib.check(lib.sf_encode_gather(
             _lib.ptr(x), x.stride(0), x.stride(1), _lib.dtype_code(x, "x"), Mx, _lib.ptr(rows), _lib.ptr(n_rows),
             row_off, _lib.ptr(W_enc), W_enc.stride(0), W_enc.stride(1), w_code,
