@@ -146,6 +146,39 @@ __device__ __forceinline__ void wave_scan16(int c, int lane, int& prefix, int& t
   }
 }
 
+// Ascending bitonic sort of the wavefront's 64 * R keys, key r*64 + lane in v[r]: exchanges
+// across lanes with xor shuffles, across registers within a lane.
+template <int R>
+__device__ __forceinline__ void wave_bitonic_sort(uint64_t (&v)[R], int lane) {
+#pragma unroll
+  for (int k = 2; k <= 64 * R; k <<= 1) {
+#pragma unroll
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      if (j >= 64) {
+        const int jr = j / 64;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          if (r & jr) continue;
+          const bool asc = ((r * 64 + lane) & k) == 0;
+          const uint64_t a = v[r], b = v[r | jr];
+          const bool sw = asc ? a > b : a < b;
+          v[r] = sw ? b : a;
+          v[r | jr] = sw ? a : b;
+        }
+      } else {
+        const bool low = (lane & j) == 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const uint64_t a = v[r];
+          const uint64_t b = (uint64_t)__shfl_xor((unsigned long long)a, j);
+          const bool asc = ((r * 64 + lane) & k) == 0;
+          v[r] = (low == asc) ? (a < b ? a : b) : (a < b ? b : a);
+        }
+      }
+    }
+  }
+}
+
 // In-place bitonic sort of s[0..P) (P a power of two) by the threads of one block
 // (nthreads threads, t = threadIdx.x), descending or ascending; ends with a barrier.
 __device__ __forceinline__ void block_bitonic_sort(uint64_t* s, int P, int t, int nthreads, bool descending) {

@@ -577,39 +577,6 @@ __device__ __forceinline__ int row_candidates(const int32_t* cnt, int64_t cap, c
   return (int)(n > hi - lo ? hi - lo : n);
 }
 
-// Ascending bitonic sort of the wavefront's 64 * R keys, key r*64 + lane in v[r]: exchanges
-// across lanes with xor shuffles, across registers within a lane.
-template <int R>
-__device__ __forceinline__ void wave_bitonic_sort(uint64_t (&v)[R], int lane) {
-#pragma unroll
-  for (int k = 2; k <= 64 * R; k <<= 1) {
-#pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j >= 64) {
-        const int jr = j / 64;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          if (r & jr) continue;
-          const bool asc = ((r * 64 + lane) & k) == 0;
-          const uint64_t a = v[r], b = v[r | jr];
-          const bool sw = asc ? a > b : a < b;
-          v[r] = sw ? b : a;
-          v[r | jr] = sw ? a : b;
-        }
-      } else {
-        const bool low = (lane & j) == 0;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const uint64_t a = v[r];
-          const uint64_t b = (uint64_t)__shfl_xor((unsigned long long)a, j);
-          const bool asc = ((r * 64 + lane) & k) == 0;
-          v[r] = (low == asc) ? (a < b ? a : b) : (a < b ? b : a);
-        }
-      }
-    }
-  }
-}
-
 __global__ __launch_bounds__(256) void rows_to_csr_wave_kernel(const int32_t* cnt, const int32_t* cidx,
                                                                const char* cval, int es, int64_t cap, int64_t M,
                                                                const int64_t* indptr, int64_t nnz, int32_t* indices,
