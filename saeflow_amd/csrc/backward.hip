@@ -635,16 +635,27 @@ __device__ __forceinline__ void put_rows(const ColArgs& a, const Item& it, char*
 // dot shares are zeroed (a load past the buffer's end, as with D = 0, returns zeros). U rows
 // in flight. Surplus waves (the grid may be sized by a bound of the item count) return at once.
 template <int DT, bool VEC, int U, bool DEC, int G, bool LIST>
-__global__ __launch_bounds__(256) void backward_units_kernel(ColArgs a, int nslab) {
+__global__ __launch_bounds__(256) void backward_units_kernel(ColArgs a, int nslab, int slab_major) {
   constexpr int ES = DT == SF_F32 ? 4 : 2, EPC = 16 / ES;
   static_assert(!DEC || U == 8, "phase A reduces 8 entries at once");
   static_assert(DEC != LIST && (!LIST || G == 1), "phase A walks the item table, phase B the slots");
   const int lane = threadIdx.x & 63;
-  const uint32_t wid = blockIdx.x * WPB + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t grp = wid / (uint32_t)nslab;
-  const int64_t slab = wid - grp * (uint32_t)nslab;
   const int64_t n_items = LIST ? min(a.n_slots, a.part_off[a.N]) : min(a.n_items, a.item_off[a.N]);
-  const int64_t i0 = (int64_t)grp * G;
+  int64_t slab, i0;
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (slab_major) {
+    // (slab, block of WPB groups) units, slab by slab, XCD x (workgroup ids b = x mod 8) taking the
+    // x-th eighth: the rows that an XCD gathers at a time are one slab's, 1 KB of each
+    const uint32_t nb = (uint32_t)(((n_items + G - 1) / G + WPB - 1) / WPB), units = nb * (uint32_t)nslab;
+    const uint32_t per = (units + 7) / 8, loc = blockIdx.x >> 3, unit = (blockIdx.x & 7) * per + loc;
+    if (loc >= per || unit >= units) return;  // whole workgroup
+    slab = unit / nb;
+    i0 = ((int64_t)(unit % nb) * WPB + wv) * G;
+  } else {  // a group's slabs side by side
+    const uint32_t wid = blockIdx.x * WPB + wv, grp = wid / (uint32_t)nslab;
+    slab = wid - grp * (uint32_t)nslab;
+    i0 = (int64_t)grp * G;
+  }
   if (i0 >= n_items) return;
   const int ni = (int)min((int64_t)G, n_items - i0);
   // the wave's items, head first: column, end of its entries, fp32 partial slot (-1: the item
@@ -1404,10 +1415,16 @@ constexpr int units_per_wave(int64_t nnz, int64_t N) { return nnz < 4 * N ? 4 : 
 
 template <int DT, bool VEC, bool DEC, int G>
 void launch_units_g(const ColArgs& a, int64_t nslab, hipStream_t s) {
-  const int64_t units = ((DEC ? a.n_items : a.n_slots) + G - 1) / G * nslab;
-  if (units == 0) return;
-  hipLaunchKernelGGL((backward_units_kernel<DT, VEC, 8, DEC, G, !DEC>), dim3((unsigned)((units + WPB - 1) / WPB)),
-                     dim3(256), 0, s, a, (int)nslab);
+  const int64_t nb = (((DEC ? a.n_items : a.n_slots) + G - 1) / G + WPB - 1) / WPB;  // a bound
+  if (nb == 0) return;
+  // Slab-major where an item gathers enough rows to reuse a slab from L2: always in phase B (columns of
+  // more than HEAVY entries; bf16 d_in 2304, us: 4096 tokens of d_sae 16384 76 -> 57, 16384 tokens 515 ->
+  // 444, of 65536 304 -> 261), in phase A from 8 entries a feature on (198 -> 191, 726 -> 693, 761 ->
+  // 752); with 4 it is even to 1% slower, with 0.5 (2^20 features) 13% slower, as a feature's W_dec
+  // and dW_dec rows then stream in 1-KB pieces.
+  const int slab_major = !DEC || (G == 1 && a.nnz >= 8 * a.N);
+  hipLaunchKernelGGL((backward_units_kernel<DT, VEC, 8, DEC, G, !DEC>), dim3((unsigned)((nb * nslab + 7) / 8 * 8)),
+                     dim3(256), 0, s, a, (int)nslab, slab_major);
 }
 
 // phase A over every work item, phase B over the heavy columns' items (one per wave)
