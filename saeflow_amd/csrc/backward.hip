@@ -888,8 +888,8 @@ __device__ __forceinline__ int64_t readlane_i64(int64_t v, int l) {
 // are loaded once for all slabs. VEC gathers as backward_units_kernel does.
 constexpr int TJ = 64, TILE_WAVES = 16, TILE_CPW = TJ / TILE_WAVES, TILE_THREADS = 64 * TILE_WAVES;
 template <int DT, bool VEC>
-__global__ __launch_bounds__(TILE_THREADS, VEC ? 8 : 4) void enc_tile_kernel(ColArgs a, int nslab, int out_vec,
-                                                                     int dec_vec) {
+__global__ __launch_bounds__(TILE_THREADS, VEC ? 8 : 4) void enc_tile_kernel(ColArgs a, int nslab, int slabs,
+                                                                                   int out_vec, int dec_vec) {
   constexpr int ES = DT == SF_F32 ? 4 : 2, EPC = 16 / ES, SD = 64 * EPC, U = 4;  // U: 64 VGPRs for 32 waves a CU
   typedef typename std::conditional<ES == 4, uint32_t, u16>::type T;
   __shared__ u32x4 tile[TJ * 64];
@@ -952,7 +952,9 @@ __global__ __launch_bounds__(TILE_THREADS, VEC ? 8 : 4) void enc_tile_kernel(Col
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)a.xs, (short)0, (int)(uint32_t)span,
                                                                      (int)BUF_W3);
   const bool full_cols = out_vec && j0 + TJ <= a.N;
-  for (int slab = 0; slab < nslab; ++slab) {
+  // grid y: the block's slabs
+  const int slab1 = min(nslab, ((int)blockIdx.y + 1) * slabs);
+  for (int slab = (int)blockIdx.y * slabs; slab < slab1; ++slab) {
     const int64_t c = (int64_t)slab * 64 + lane;
     const bool cin = c < nch;
     const uint32_t coff = (uint32_t)(min(c, max(nch - 1, (int64_t)0)) * 16);
@@ -1439,11 +1441,20 @@ void launch_units(const ColArgs& a, int64_t nslab, hipStream_t s) {
   launch_units_g<DT, VEC, DEC, 1>(a, nslab, s);
 }
 
+// enc_tile_kernel's blocks: below this many column tiles the slabs are split over blocks. Two blocks
+// share a CU, and a tile's slabs one after the other left most of them idle (bf16 d_in 2304, us, whole
+// tiles -> split: d_sae 16384, 1024 tokens 96 -> 48, 4096 tokens 137 -> 92; 65536, 16384 tokens 434 -> 371,
+// a bound of 2048 blocks 398). At 2^20 features the split is slower (1644 -> 1959): the tiles fill the
+// chip by themselves and each block reads its columns' bounds again.
+constexpr int64_t TILE_BLOCKS = 8192;
 template <int DT>
 void launch_tile(const ColArgs& a, bool vec, int out_vec, int dec_vec, int64_t nslab, hipStream_t s) {
-  const dim3 grid((unsigned)(((a.N + TJ - 1) / TJ + 31) / 32 * 32));
-  if (vec) hipLaunchKernelGGL((enc_tile_kernel<DT, true>), grid, dim3(TILE_THREADS), 0, s, a, (int)nslab, out_vec, dec_vec);
-  else hipLaunchKernelGGL((enc_tile_kernel<DT, false>), grid, dim3(TILE_THREADS), 0, s, a, (int)nslab, out_vec, dec_vec);
+  const int64_t tiles = (a.N + TJ - 1) / TJ;
+  const int64_t split = std::min(nslab, std::max<int64_t>(1, (TILE_BLOCKS + tiles - 1) / tiles));
+  const int slabs = (int)((nslab + split - 1) / split);
+  const dim3 grid((unsigned)((tiles + 31) / 32 * 32), (unsigned)((nslab + slabs - 1) / slabs));
+  if (vec) hipLaunchKernelGGL((enc_tile_kernel<DT, true>), grid, dim3(TILE_THREADS), 0, s, a, (int)nslab, slabs, out_vec, dec_vec);
+  else hipLaunchKernelGGL((enc_tile_kernel<DT, false>), grid, dim3(TILE_THREADS), 0, s, a, (int)nslab, slabs, out_vec, dec_vec);
 }
 
 template <bool DEC>
