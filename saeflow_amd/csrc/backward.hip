@@ -503,6 +503,7 @@ struct ColArgs {
   float* d_benc;  // [N]
   float* part;    // [slots, 2, D] fp32, then [slots] fp32 for b_enc
   int64_t n_slots;
+  const int4* rec;  // [n_items] what a wave needs of each work item (item_records_kernel), or NULL
 };
 
 // x' = cast_DT(fp32(x) - fp32(b_dec)), the forward's MFMA operand (encode.py:72), [M, D]
@@ -566,6 +567,23 @@ __device__ __forceinline__ Item item_at(const ColArgs& a, int64_t item) {
   it.e_hi = min(c_hi, it.e_lo + CHUNK);
   it.slots = a.part_off[it.j + 1] - a.part_off[it.j];
   return it;
+}
+
+// A work item in one load: {column, first entry, end of its entries, slot}, slot = its partial slot in
+// a column of several items, -1 without one, -2 - slot for the only item of a heavy column. A wave of
+// backward_units_kernel walks a chain of dependent loads before its first gather (item -> column ->
+// bounds -> entries -> rows); the record takes two links out of it (dW_dec sums, us: 2^20 features 763 ->
+// 686, fp32 777 tokens of 768 x 8192 17.3 -> 15.7; within 2% where a feature has 16 entries). The grid also
+// zeroes g_pre, which entries outside [0, N) keep.
+__global__ __launch_bounds__(256) void item_records_kernel(ColArgs a, int4* rec) {
+  const int64_t t0 = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+  for (int64_t i = t0; i < a.nnz; i += step) a.g_pre[i] = 0.f;
+  const int64_t n = min(a.n_items, a.item_off[a.N]);
+  for (int64_t i = t0; i < n; i += step) {
+    const Item it = item_at(a, i);
+    const int slot = (int)(a.part_off[it.j] + it.q);
+    rec[i] = make_int4((int)it.j, (int)it.e_lo, (int)it.e_hi, it.slots > 1 ? slot : (it.slots == 1 ? -2 - slot : -1));
+  }
 }
 
 template <int DT>
@@ -668,13 +686,25 @@ __global__ __launch_bounds__(256) void backward_units_kernel(ColArgs a, int nsla
     q_slot[g] = -1;
     q_end[g] = 0;
     if (g < ni) {
-      const Item it = item_at(a, LIST ? (int64_t)a.slot_item[i0 + g] : i0 + g);
-      q_j[g] = (int)it.j;
+      const int64_t item = LIST ? (int64_t)a.slot_item[i0 + g] : i0 + g;
+      int64_t lo;
       // phase A stores the row of a one-item column directly; phase B always fills the slot
-      q_slot[g] = it.slots > (DEC ? 1 : 0) ? (int)(a.part_off[it.j] + it.q) : -1;
-      q_end[g] = it.e_hi;
-      if (g == 0) e_lo = it.e_lo;
-      e_hi = it.e_hi;
+      if (a.rec) {
+        const int4 q = a.rec[item];
+        q_j[g] = __builtin_amdgcn_readfirstlane(q.x);
+        lo = __builtin_amdgcn_readfirstlane(q.y);
+        q_end[g] = __builtin_amdgcn_readfirstlane(q.z);
+        const int slot = __builtin_amdgcn_readfirstlane(q.w);
+        q_slot[g] = slot >= 0 ? slot : (DEC ? -1 : -2 - slot);
+      } else {
+        const Item it = item_at(a, item);
+        q_j[g] = (int)it.j;
+        lo = it.e_lo;
+        q_end[g] = it.e_hi;
+        q_slot[g] = it.slots > (DEC ? 1 : 0) ? (int)(a.part_off[it.j] + it.q) : -1;
+      }
+      if (g == 0) e_lo = lo;
+      e_hi = q_end[g];
     }
   }
   const int64_t nch = (a.D + EPC - 1) / EPC, c = slab * 64 + lane;
@@ -1652,7 +1682,7 @@ extern "C" int sf_backward_columns(const int64_t* colptr, const int32_t* csc_row
                (long long)work_floats, (long long)((nslab + 1) * nnz));
   }
   hipStream_t s = (hipStream_t)stream;
-  if (nnz > 0) {  // entries outside [0, N) keep g_pre = 0
+  if (nnz > 0 && N == 0) {  // entries outside [0, N) keep g_pre = 0
     hipLaunchKernelGGL(fill_i32_kernel, dim3((unsigned)std::min<int64_t>(4096, (nnz + 255) / 256)), dim3(256), 0, s,
                        (int32_t*)g_pre, nnz, 0);
     SF_LAUNCH_CHECK("fill_i32_kernel");
@@ -1674,7 +1704,19 @@ extern "C" int sf_backward_columns(const int64_t* colptr, const int32_t* csc_row
   const bool vec = D % (16 / es) == 0 && aligned16(xs, sx, es) && aligned16(g_xhat, sg, es) &&
                    aligned16(w_dec, sw, es) && aligned16(d_wdec, D, es) &&
                    span_x < (1LL << 32) && span_g < (1LL << 32);  // the per-row gathers are buffer loads
+  // the records sit in d_wenc, which enc_tile_kernel overwrites once the units are done with them
+  a.rec = nullptr;
   if (nnz > 0) {
+    if (D * N * es >= max_items * (int64_t)sizeof(int4) && (uintptr_t)d_wenc % 16 == 0) {
+      hipLaunchKernelGGL(item_records_kernel, dim3((unsigned)std::min<int64_t>(GRID_BLOCKS, (std::max(nnz, max_items) + 255) / 256)),
+                         dim3(256), 0, s, a, (int4*)d_wenc);
+      SF_LAUNCH_CHECK("item_records_kernel");
+      a.rec = (const int4*)d_wenc;
+    } else {
+      hipLaunchKernelGGL(fill_i32_kernel, dim3((unsigned)std::min<int64_t>(4096, (nnz + 255) / 256)), dim3(256), 0, s,
+                         (int32_t*)g_pre, nnz, 0);
+      SF_LAUNCH_CHECK("fill_i32_kernel");
+    }
     launch_units_dt<true>(a, dt, vec, nslab, s);
     SF_LAUNCH_CHECK("backward_units_kernel (dW_dec)");
     hipLaunchKernelGGL(gpre_kernel, dim3((unsigned)std::min<int64_t>(GRID_BLOCKS, (nnz + 255) / 256)), dim3(256), 0, s,
