@@ -225,6 +225,13 @@ SF_API int sf_scan_counts(const int32_t* counts, int64_t M, int64_t* indptr, voi
  * 2^20 - 1; 0 if M is 0), both int64 on the device, for the caller's one read back (decode.py:88). */
 SF_API int sf_scan_counts_stats(const int32_t* counts, int64_t M, int64_t* indptr, int64_t* stats, void* stream);
 
+/* sf_count_nonzero that also leaves the nonzeros of every row with at most cap of them, in any order, as
+ * (column, value) pairs in idx/val[m, :counts[m]] (int32 [M, cap], f_dt [M, cap]): the lists that
+ * sf_rows_to_csr places in a CSR; sf_compact_long places the other rows. Rows of f contiguous and 16-B
+ * aligned; 0 <= cap <= 256. */
+SF_API int sf_row_lists(const void* f, int64_t sfm, int64_t sfn, int f_dt, int64_t M, int64_t N, int64_t cap,
+                 int32_t* counts, int32_t* idx, void* val, void* stream);
+
 /* Compaction: for every row m, the nonzero elements of f row m, in increasing column
  * order, go to indices/values[indptr[m] ...] (canonical CSR, values copied bit-exact).
  * Replaces _compact_kernel (reference decode.py:61-74, launched at :91-93).
@@ -233,6 +240,12 @@ SF_API int sf_scan_counts_stats(const int32_t* counts, int64_t M, int64_t* indpt
 SF_API int sf_compact(const void* f, int64_t sfm, int64_t sfn, int f_dt, int64_t M, int64_t N,
                const int64_t* indptr, int64_t nnz, int32_t* indices, void* values,
                void* stream);
+
+/* sf_compact of the rows longer than longer_than alone; the segments of the others stay as they are.
+ * Rows of f contiguous and 16-B aligned unless longer_than is 0 (every row). */
+SF_API int sf_compact_long(const void* f, int64_t sfm, int64_t sfn, int f_dt, int64_t M, int64_t N,
+                    const int64_t* indptr, int64_t nnz, int64_t longer_than, int32_t* indices, void* values,
+                    void* stream);
 
 /* Sparse decode: out[m] = b_dec + sum_{j in row m} values[j] * W_dec[indices[j]],
  * fp32 accumulation. Replaces _decode_kernel (reference decode.py:28-55) launched by

@@ -44,9 +44,11 @@ SIGNATURES = {
     "sf_rows_to_csr_bounded": (_I32, [_P, _P, _P, _I32, _I64, _I64, _P, _I64, _I64, _P, _P, _P]),
     "sf_rows_topk": (_I32, [_P, _P, _P, _I32, _I64, _I64, _I64, _I64, _P, _P, _P]),
     "sf_count_nonzero": (_I32, [_P, _I64, _I64, _I32, _I64, _I64, _P, _P]),
+    "sf_row_lists": (_I32, [_P, _I64, _I64, _I32, _I64, _I64, _I64, _P, _P, _P, _P]),
     "sf_scan_counts": (_I32, [_P, _I64, _P, _P]),
     "sf_scan_counts_stats": (_I32, [_P, _I64, _P, _P, _P]),
     "sf_compact": (_I32, [_P, _I64, _I64, _I32, _I64, _I64, _P, _I64, _P, _P, _P]),
+    "sf_compact_long": (_I32, [_P, _I64, _I64, _I32, _I64, _I64, _P, _I64, _I64, _P, _P, _P]),
     "sf_decode": (_I32, [_P, _P, _P, _I32, _I64, _P, _I64, _I64, _I32, _I64, _P, _I32, _P, _I64, _I64,
                          _I32, _I64, _I64, _P, _P]),
     "sf_topk": (_I32, [_P, _I64, _I64, _I32, _I64, _I64, _I64, _P, _P, _P]),

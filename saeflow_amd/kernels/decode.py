@@ -55,16 +55,55 @@ def scan_counts(row_nnz):
 def compact(f, indptr, nnz):
     """(indices int32 [nnz], values [nnz]): the nonzeros of every row of f in column order,
     placed at indptr[row] (_compact_kernel, decode.py:61-74)."""
-    M, N = f.shape
-    dev = _lib.require_gpu(("f", f), ("indptr", indptr))
     indices = torch.empty(nnz, dtype=torch.int32, device=f.device)
     values = torch.empty(nnz, dtype=f.dtype, device=f.device)
+    compact_into(f, indptr, nnz, 0, indices, values)
+    return indices, values
+
+
+def compact_into(f, indptr, nnz, longer_than, indices, values):
+    """compact() of the rows of more than longer_than nonzeros, into their segments."""
+    M, N = f.shape
+    dev = _lib.require_gpu(("f", f), ("indptr", indptr))
     if nnz and M:
         with _lib.device(dev):
-            _lib.check(_lib.load().sf_compact(_lib.ptr(f), f.stride(0), f.stride(1), _lib.dtype_code(f, "f"), M, N,
-                                              _lib.ptr(indptr), nnz, _lib.ptr(indices), _lib.ptr(values),
-                                              _lib.stream(dev)))
-    return indices, values
+            _lib.check(_lib.load().sf_compact_long(_lib.ptr(f), f.stride(0), f.stride(1), _lib.dtype_code(f, "f"), M, N,
+                                                   _lib.ptr(indptr), nnz, longer_than, _lib.ptr(indices),
+                                                   _lib.ptr(values), _lib.stream(dev)))
+
+
+LIST_CAP = 256  # nonzeros of a row that row_lists keeps: what rows_to_csr sorts in one wavefront
+# dense_to_csr without counts reads f once, through lists, from these sizes on. Measured (us, bf16,
+# counts + compaction -> lists): 16384 x 65536 16 nonzeros a row 641 -> 361, 64 655 -> 388, 200 760 -> 471; 512 x
+# 2^20 64 a row 323 -> 187; 16384 x 16384 209 -> 135, 225 -> 178 at 200 a row. Where every row is longer than its
+# list, the second read comes on top of the lists' work: 300 a row 788 -> 794 (2 GiB of f), 226 -> 237 (512 MiB),
+# 600 a row 812 -> 818 and 236 -> 239. Of smaller f that share grows (f of 64 MiB, 64 a row: 49 either way), so they
+# keep the two passes, as do rows under 32 KiB, where the sort of the lists weighs more (16384 x 4096, 200 a row:
+# 100 -> 113).
+LIST_MIN_BYTES = 1 << 29
+LIST_MIN_ROW_BYTES = 1 << 15
+
+
+def row_lists(f):
+    """(counts int32 [M], idx int32 [M, LIST_CAP], val [M, LIST_CAP]): row_counts(f) and the nonzeros
+    of every row with at most LIST_CAP of them, in no particular order, from one read of f. Rows of f
+    must be contiguous and 16-B aligned."""
+    M, N = f.shape
+    dev = _lib.require_gpu(("f", f))
+    counts = torch.empty(M, dtype=torch.int32, device=f.device)
+    idx = torch.empty(M, LIST_CAP, dtype=torch.int32, device=f.device)
+    val = torch.empty(M, LIST_CAP, dtype=f.dtype, device=f.device)
+    if M:
+        with _lib.device(dev):
+            _lib.check(_lib.load().sf_row_lists(_lib.ptr(f), f.stride(0), f.stride(1), _lib.dtype_code(f, "f"), M, N,
+                                                LIST_CAP, _lib.ptr(counts), _lib.ptr(idx), _lib.ptr(val),
+                                                _lib.stream(dev)))
+    return counts, idx, val
+
+
+def _vec_rows(f):
+    """Rows that the 16-B loads take (csr.hip's vec_rows)."""
+    return f.stride(1) == 1 and f.data_ptr() % 16 == 0 and f.stride(0) * f.element_size() % 16 == 0
 
 
 def dense_to_csr(f, row_nnz=None):
@@ -77,6 +116,16 @@ def dense_to_csr(f, row_nnz=None):
     M, N = f.shape
     _lib.require_gpu(("f", f), ("row_nnz", row_nnz))
     _lib.dtype_code(f, "f")
+    row_bytes = N * f.element_size()
+    if row_nnz is None and row_bytes >= LIST_MIN_ROW_BYTES and M * row_bytes >= LIST_MIN_BYTES and _vec_rows(f):
+        row_nnz, idx, val = row_lists(f)
+        indptr, nnz, longest = scan_counts(row_nnz)
+        if nnz > M * LIST_CAP * 9 // 8:  # nearly all rows are longer than their list
+            return indptr, *compact(f, indptr, nnz)
+        indices, values = rows_to_csr(row_nnz, idx, val, indptr, nnz, min(longest, LIST_CAP))
+        if longest > LIST_CAP:  # a second read of the rows that are longer than their list
+            compact_into(f, indptr, nnz, LIST_CAP, indices, values)
+        return indptr, indices, values
     if row_nnz is None:
         row_nnz = row_counts(f)
     elif row_nnz.numel() != M:

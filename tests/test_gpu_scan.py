@@ -4,7 +4,8 @@ it leaves for the host, and the row-candidate calls that use them."""
 import pytest
 import torch
 
-from saeflow_amd.kernels import encode_rows, exclusive_scan, rows_to_csr, scan_counts
+from saeflow_amd import kernels
+from saeflow_amd.kernels import dense_to_csr, encode_rows, exclusive_scan, row_lists, rows_to_csr, scan_counts
 
 pytestmark = pytest.mark.gpu
 
@@ -51,3 +52,44 @@ def test_row_candidates_count_from_zero_and_sort_with_a_known_bound(M):
         assert (longest > 256) == (b > 0)
         for a, c in zip(rows_to_csr(cnt, idx, val, indptr, nnz, longest), rows_to_csr(cnt, idx, val, indptr, nnz)):
             assert torch.equal(a, c)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N", [8, 2048, 2051, 16384, 16392, 40003])  # rows of one group of loads, of several, with a tail
+def test_dense_to_csr_counts_and_lists_in_one_read(dtype, N, monkeypatch):
+    """Without counts: rows that fit their lists (up to 256 nonzeros) and batches with some that do
+    not, against the CSR by hand; -0.0 is a zero, NaN and infinities are kept. The lists are for large
+    f alone, so the sizes they start at are lowered here."""
+    monkeypatch.setattr(kernels.decode, "LIST_MIN_BYTES", 0)
+    monkeypatch.setattr(kernels.decode, "LIST_MIN_ROW_BYTES", 0)
+    M, pad = 5, -N % 8
+    for longest in (0, 1, 255, 256, 257, N):
+        longest = min(longest, N)
+        f = torch.zeros(M, N + pad, dtype=dtype)[:, :N]  # rows stay 16-B aligned
+        for m, n in enumerate((longest, longest // 2, 0, min(longest, 3), longest)):
+            g = torch.Generator().manual_seed(7 * m + n)
+            f[m, torch.randperm(N, generator=g)[:n]] = torch.rand(n, generator=g).to(dtype) + 1
+        if longest >= 3:
+            f[3, f[3].nonzero().flatten()] = torch.tensor([float("nan"), float("-inf"), -2.0], dtype=dtype)
+        f[2, N - 1] = -0.0
+        dev = torch.empty(M, N + pad, dtype=dtype, device="cuda")[:, :N].copy_(f)
+        counts = (f != 0).sum(1)
+        lists, idx, val = row_lists(dev)
+        assert torch.equal(lists.cpu(), counts.int())
+        indptr, indices, values = dense_to_csr(dev)
+        where = (f != 0).nonzero()
+        assert torch.equal(indptr.cpu(), torch.cat([torch.zeros(1, dtype=torch.int64), counts.cumsum(0)]))
+        assert torch.equal(indices.cpu(), where[:, 1].int())
+        bits = torch.int32 if dtype == torch.float32 else torch.int16
+        assert torch.equal(values.cpu().view(bits), f[where[:, 0], where[:, 1]].view(bits))
+
+
+def test_dense_to_csr_of_rows_the_vector_loads_do_not_take(monkeypatch):
+    monkeypatch.setattr(kernels.decode, "LIST_MIN_BYTES", 0)
+    monkeypatch.setattr(kernels.decode, "LIST_MIN_ROW_BYTES", 0)
+    f = torch.zeros(4, 1001).index_fill_(1, torch.tensor([0, 17, 1000]), 2.5).cuda()
+    for g in (f, f[:, 1:], f.t().contiguous().t()):
+        indptr, indices, values = dense_to_csr(g)
+        want = g.to_sparse_csr()
+        assert torch.equal(indptr, want.crow_indices()) and torch.equal(indices.long(), want.col_indices())
+        assert torch.equal(values, want.values())
