@@ -34,6 +34,8 @@ class SparseSAEFunction(torch.autograd.Function):
         x_hat = ops.decode_sparse(sae, (indptr, indices, values))
         ctx.save_for_backward(x, W_enc, b_enc, W_dec, b_dec, indptr, indices, values)
         ctx.mark_non_differentiable(indptr, indices)
+        # absent gradients arrive as None, not as zeros filled for indptr, indices and an unused output
+        ctx.set_materialize_grads(False)
         return x_hat, indptr, indices, values
 
     @staticmethod
