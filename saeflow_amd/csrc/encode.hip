@@ -263,9 +263,9 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
   if (swn == 1 && swk >= N && (N % epc) == 0 && ((swk * esz) % 16) == 0 && aligned(w, 16) &&
       (int64_t)bk * swk * esz + N * esz < (1LL << 31))
     wp = W_NMAJOR;
-  // (K * esz a multiple of 4: a buffer load drops the dword that the range ends inside, which would
-  // lose the last d_in element of a tile's last feature)
-  else if (swk == 1 && swn >= K && ((swn * esz) % 16) == 0 && aligned(w, 16) && ((K * esz) % 4) == 0 &&
+  // (K in whole 16-B chunks: a chunk that straddles K would bring in what lies behind the row, its
+  // padding or a parent tensor's columns; x' is zero there, but 0 * NaN is not)
+  else if (swk == 1 && swn >= K && ((swn * esz) % 16) == 0 && aligned(w, 16) && (K % epc) == 0 &&
            (int64_t)BN * swn * esz + K * esz < (1LL << 31))
     wp = W_KMAJOR;
   const int sw = slim_w(wp, swk, swn);

@@ -199,7 +199,8 @@ def test_fused_encode_odd_d_in_of_a_padded_transposed_weight(dtype):
     """A d_in-contiguous W_enc whose rows are padded to 16 B and end inside a dword (odd d_in in 16
     bits): the last d_in element of every feature counts, the last feature of a tile included."""
     M, d_in, d_sae = 3, 777, 300
-    back = torch.zeros(d_sae, 784, dtype=dtype)
+    back = torch.full((d_sae, 784), float("nan"), dtype=dtype)  # padded with anything
+    back[:, :d_in] = 0
     back[:, d_in - 1] = torch.arange(1, d_sae + 1).to(dtype)
     x = torch.zeros(M, d_in, dtype=dtype)
     x[:, d_in - 1] = 1

@@ -9,7 +9,7 @@ registers)."""
 import pytest
 import torch
 
-from saeflow_amd.kernels import encode_pre, encode_rows, fused_encode
+from saeflow_amd.kernels import encode_gather, encode_pre, encode_rows, fused_encode
 
 pytestmark = pytest.mark.gpu
 
@@ -37,8 +37,8 @@ def make(shape, dtype, layout, nan=False):
     W = (torch.randn(K, N, generator=g) / K ** 0.5).to(dtype).cuda()
     if layout == "features":
         pass
-    elif layout == "d_in":  # rows padded to 16 B, as an aligned transposed view has them
-        back = torch.zeros(N, -(-K // 8) * 8, dtype=dtype, device="cuda")
+    elif layout == "d_in":  # rows padded to 16 B, as an aligned transposed view has them, with anything
+        back = torch.full((N, -(-K // 8) * 8), float("nan"), dtype=dtype, device="cuda")
         back[:, :K] = W.T
         W = back.T[:K]
     elif layout == "odd_features":  # rows of odd length
@@ -62,7 +62,7 @@ def aligned(shape, dtype, layout):
     M, K, N = shape
     if layout == "features":
         return N % (4 if dtype == torch.float32 else 8) == 0
-    return layout == "d_in" and (K % 2 == 0 or dtype == torch.float32)
+    return layout == "d_in" and K % (4 if dtype == torch.float32 else 8) == 0
 
 
 def same(a, b):
@@ -90,6 +90,31 @@ def test_small_tiles_equal_the_wide_tile(dtype, layout, tile):
             assert torch.equal(*counts), (shape, act)
         got, want = (encode_pre(x, W, p["b_enc"], p["b_dec"], config=c) for c in (config(tile, dtype), wide(dtype)))
         assert same(got, want), shape
+
+
+@pytest.mark.parametrize("d_in", [1001, 1002, 1004, 1006, 70, 9])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_padding_behind_d_in_stays_out_of_the_features(dtype, d_in):
+    """A d_in-contiguous W_enc with 16-B aligned rows that end inside a chunk, NaN behind them: the
+    features are those of the dense weight on every path."""
+    M, N = 130, 300
+    x, W, p, cut = make((M, d_in, N), dtype, "features")
+    padded = make((M, d_in, N), dtype, "d_in")[1]
+    assert torch.equal(padded, W) and padded.stride(0) == 1 and padded.stride(1) % 8 == 0
+    want = fused_encode(x, W, p["b_enc"], p["b_dec"], cut, "jumprelu", config=wide(dtype))
+    assert not want.isnan().any()
+    bk = wide(dtype)["BLOCK_K"]
+    for c in (None, wide(dtype), {**wide(dtype), "NUM_WAVES": 4}, config(TILES[0], dtype),
+              {"BLOCK_M": 256, "BLOCK_N": 128, "BLOCK_K": bk // 2}):
+        assert same(fused_encode(x, padded, p["b_enc"], p["b_dec"], cut, "jumprelu", config=c), want), c
+    rows, n = torch.arange(M, dtype=torch.int32, device="cuda"), torch.full((1,), M, dtype=torch.int32, device="cuda")
+    assert same(encode_gather(x, padded, p["b_enc"], p["b_dec"], rows, n, cut, "jumprelu", out_rows=M), want)
+    for c in (None, wide(dtype)):
+        cnt, idx, val = encode_rows(x, padded, p["b_enc"], p["b_dec"], cut, "jumprelu", cap=N, config=c)
+        live = torch.arange(N, device="cuda")[None] < cnt[:, None]
+        f = torch.zeros(M, N + 1, dtype=dtype, device="cuda")
+        f.scatter_(1, torch.where(live, idx, N).long(), val)
+        assert same(f[:, :N].contiguous(), want), c
 
 
 @pytest.mark.parametrize("tile", TILES)
