@@ -221,11 +221,11 @@ def encode_rows(x, W_enc, b_enc, b_dec, threshold=None, activation="relu", *, ca
     if K != K_w:
         raise ValueError(f"x has d_in={K} but W_enc has d_in={K_w}")
     vdt = out_dtype or x.dtype
-    # with features to encode, the call clears the counts itself
+    # with features to encode, the call clears the counts itself (without, it checks its arguments)
     cnt = (torch.empty if N else torch.zeros)(M, device=x.device, dtype=torch.int32)
     idx = torch.empty(M, cap, device=x.device, dtype=torch.int32)
     val = torch.empty(M, cap, device=x.device, dtype=vdt)
-    if M == 0 or N == 0:
+    if M == 0:
         return cnt, idx, val
     threshold = threshold if activation == "jumprelu" else None
     dev = _lib.require_gpu(("x", x), ("W_enc", W_enc), ("b_enc", b_enc), ("b_dec", b_dec),
@@ -242,8 +242,9 @@ def encode_rows(x, W_enc, b_enc, b_dec, threshold=None, activation="relu", *, ca
     lib = _lib.load()
     w_code = _lib.dtype_code(W_enc, "W_enc")
     ws = torch.empty(max(_lib.encode_workspace_bytes(M, K, w_code), 16), dtype=torch.uint8, device=x.device)
+    encode = lib.sf_encode_rows_cleared if N else lib.sf_encode_rows
     with _lib.device(dev):
-        _lib.check(lib.sf_encode_rows_cleared(
+        _lib.check(encode(
             _lib.ptr(x), x.stride(0), x.stride(1), _lib.dtype_code(x, "x"),
             _lib.ptr(W_enc), W_enc.stride(0), W_enc.stride(1), w_code,
             _lib.ptr(b_enc), _lib.dtype_code(b_enc, "b_enc"), _lib.ptr(b_dec), _lib.dtype_code(b_dec, "b_dec"),

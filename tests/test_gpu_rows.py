@@ -309,6 +309,20 @@ def test_encode_gather_equals_the_dense_encode_of_the_rows(dtype):
         assert _bits_equal(got[:k], want[sel]), (live, off, R)
 
 
+def test_encode_rows_without_features_checks_its_operands():
+    x, W = torch.randn(5, 8, device="cuda"), torch.empty(8, 0, device="cuda")
+    none, b = torch.empty(0, device="cuda"), torch.zeros(8, device="cuda")
+    for bad in (dict(b_enc=none, b_dec=b[:7]), dict(b_enc=b, b_dec=b)):
+        with pytest.raises(ValueError, match="must have shape"):
+            encode_rows(x, W, bad["b_enc"], bad["b_dec"], cap=4)
+    with pytest.raises(ValueError, match="row_floor"):
+        encode_rows(x, W, none, b, cap=4, row_floor=torch.zeros(4, device="cuda"))
+    with pytest.raises(ValueError, match="capacity"):
+        encode_rows(x, W, none, b, cap=5000)
+    cnt, idx, val = encode_rows(x, W, none, b, cap=4)
+    assert cnt.tolist() == [0] * 5 and idx.shape == val.shape == (5, 4)
+
+
 def test_encode_gather_rows_outside_x_encode_a_zero_row():
     # A row id outside [0, Mx) encodes a zero x' row, which is what a token equal to b_dec gives:
     # x' = cast(fp32(b_dec) - fp32(b_dec)) = 0.

@@ -142,6 +142,14 @@ def test_gathered_entry_points_validate_before_any_launch():
     assert lib.sf_overflow_rows(16, 8, -1, 16, 16, None) == _lib.SF_EINVAL
 
 
+def test_encode_rows_without_features_still_checks_its_operands():
+    from saeflow_amd.kernels import encode_rows
+    x, W, b = torch.zeros(3, 8), torch.zeros(8, 0), torch.zeros(8)
+    with pytest.raises(ValueError, match="GPU"):
+        encode_rows(x, W, torch.zeros(0), b, cap=4)
+    assert encode_rows(x[:0], W, torch.zeros(0), b, cap=4)[0].shape == (0,)  # no tokens: nothing to run
+
+
 def test_best_config_is_none_before_a_tuned_launch():
     from saeflow_amd.kernels import best_config
     from saeflow_amd.kernels import encode as kenc
