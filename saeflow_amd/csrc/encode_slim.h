@@ -67,6 +67,12 @@ __device__ __forceinline__ void wait_vmcnt() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
+// Memory operations stay on their side of it, in the compiler's passes and its scheduler.
+__device__ __forceinline__ void order_vmem() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // LDS layouts, conflict free on 64 banks of 4 B (encode_kernels.h's swizzles for other row
 // lengths). x' and a K-contiguous W: rows of KC chunks.
 template <int KC>
@@ -224,7 +230,7 @@ __device__ __forceinline__ void slim_dense(const GemmArgs& a, f32x16 (&acc)[NB][
 // go from registers to LDS at step kt and those of kt + 3 are loaded (two sets of registers); x'
 // stays on DMA, two steps ahead.
 template <int DT, int SW, typename TL, int EPI, int AUX>
-__global__ __launch_bounds__(TL::NT, TL::NW / 2 > 2 ? 2 : (TL::ST * TL::NS > 81920 ? TL::NW / 4 : TL::NW / 2)) void gemm_slim_kernel(GemmArgs a) {
+__global__ __launch_bounds__(TL::NT, TL::ST * TL::NS > 81920 ? TL::NW / 4 : TL::NW / 2) void gemm_slim_kernel(GemmArgs a) {
   constexpr int E = Traits<DT>::E, EPC = Traits<DT>::EPC;
   constexpr int MB = TL::MB, NB = TL::NB, KC = TL::KC, NS = TL::NS, NW = TL::NW, TN = TL::TN, TM = TL::TM;
   constexpr int PW = TL::PW, PX = TL::PX, BK = KC * EPC, KS = KC / 2;  // KS k16 (fp32: k8) steps per K-step
@@ -445,6 +451,7 @@ __global__ __launch_bounds__(TL::NT, TL::NW / 2 > 2 ? 2 : (TL::ST * TL::NS > 819
     wait_vmcnt0();
     put_w(0, s0, rw[0]);
     load_w(2, rw[0]);
+    order_vmem();
   } else {
     issue(0, s0);
     issue(1, s1);
@@ -494,12 +501,16 @@ __global__ __launch_bounds__(TL::NT, TL::NW / 2 > 2 ? 2 : (TL::ST * TL::NS > 819
       wait_lgkmcnt0();
       barrier_no_fence();
       // This thread's x' of kt + 1 (issued a step ago) and W registers of kt + 1 (two steps ago);
-      // only the W loads of kt + 2, issued after both, may still be in flight.
+      // only the W loads of kt + 2, issued after both, may still be in flight. vmcnt counts in issue
+      // order, so a step's DMAs must all precede its W loads and none of these may slip behind the
+      // next step's wait; no data ties them, so order_vmem keeps the compiler from moving either.
       if (!narrow) wait_vmcnt<PW>();
       else wait_vmcnt0();
       put_w(kt + 1, wnx, rw[1 - ODD]);
       issue_x(kt + 2, nxt);
+      order_vmem();
       load_w(kt + 3, rw[1 - ODD]);
+      order_vmem();
     }
     Frag f[2];
     load_frag(f[0], cur, 0);
