@@ -99,6 +99,20 @@ extern "C" int sf_encode_workspace_size(int64_t M, int64_t K, int w_dt, int64_t*
 
 namespace {
 
+// The path that W's layout takes: the DMA paths, or staging through registers.
+int w_path(const void* w, int64_t swk, int64_t swn, int64_t N, int64_t K, int w_dt) {
+  const int esz = sf_dtype_size(w_dt), epc = 16 / esz, bk = bk_of(w_dt);
+  if (swn == 1 && swk >= N && (N % epc) == 0 && ((swk * esz) % 16) == 0 && aligned(w, 16) &&
+      (int64_t)bk * swk * esz + N * esz < (1LL << 31))
+    return W_NMAJOR;
+  // (K in whole 16-B chunks: a chunk that straddles K would bring in what lies behind the row, its
+  // padding or a parent tensor's columns; x' is zero there, but 0 * NaN is not)
+  if (swk == 1 && swn >= K && ((swn * esz) % 16) == 0 && aligned(w, 16) && (K % epc) == 0 &&
+      (int64_t)BN * swn * esz + K * esz < (1LL << 31))
+    return W_KMAJOR;
+  return W_GENERIC;
+}
+
 // The slim kernels' W path (encode_slim.h): the DMA paths where the 256x256 kernels have one,
 // else registers for a W that is contiguous along one axis; -1 for other strides.
 int slim_w(int wp, int64_t swk, int64_t swn) {
@@ -157,6 +171,26 @@ int pick_slim(int64_t M, int64_t N, int64_t K, int w_dt, int sw) {
   }
   return best;
 }
+
+}  // namespace
+
+extern "C" int sf_encode_tiling(int64_t M, int64_t N, int64_t K, const void* w, int64_t swk, int64_t swn, int w_dt,
+                                int32_t* cfg_out) {
+  const int rc = sf_encode_config(M, N, K, w_dt, cfg_out);
+  if (rc != SF_OK) return rc;
+  SF_REQUIRE(M >= 0 && N >= 0 && K >= 0, "sf_encode_tiling: negative size");
+  const int i = M == 0 || N == 0 ? -1 : pick_slim(M, N, K, w_dt, slim_w(w_path(w, swk, swn, N, K, w_dt), swk, swn));
+  if (i >= 0) {
+    const SlimShape q = slim_shape(i);
+    cfg_out[0] = q.tm;
+    cfg_out[1] = q.tn;
+    cfg_out[2] = q.kc * bk_of(w_dt) / 8;
+    cfg_out[4] = q.nw;
+  }
+  return SF_OK;
+}
+
+namespace {
 
 template <int DT>
 hipError_t launch_rows_o(int out_dt, bool floor, const GemmArgs& a, int wp, hipStream_t s) {
@@ -242,7 +276,7 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
   else SF_REQUIRE(cand_cnt && (cap == 0 || (cand_idx && cand_val)), "%s: NULL candidate buffer", fn);
   SF_REQUIRE(epi != EPI_ROWS_FLOOR || row_floor != nullptr, "%s: NULL row floor", fn);
   SF_REQUIRE(M <= INT32_MAX - BM && N <= INT32_MAX - BN, "%s: M or N too large", fn);
-  const int esz = sf_dtype_size(w_dt), epc = 16 / esz;
+  const int esz = sf_dtype_size(w_dt);
   const int64_t Kp = padded_k(K, w_dt);
   SF_REQUIRE(Kp * esz * BM < (1LL << 31), "%s: d_in=%lld too large for 32-bit tile offsets", fn, (long long)K);
   const int64_t need = workspace_bytes_of(M, K, w_dt);
@@ -258,16 +292,7 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
   a.out = out; a.som = som; a.son = son; a.out_dt = out_dt;
   a.row_nnz = row_nnz; a.M = M; a.N = N; a.K = K; a.act = act;
 
-  // W layouts the DMA paths take; anything else is staged through registers
-  int wp = W_GENERIC;
-  if (swn == 1 && swk >= N && (N % epc) == 0 && ((swk * esz) % 16) == 0 && aligned(w, 16) &&
-      (int64_t)bk * swk * esz + N * esz < (1LL << 31))
-    wp = W_NMAJOR;
-  // (K in whole 16-B chunks: a chunk that straddles K would bring in what lies behind the row, its
-  // padding or a parent tensor's columns; x' is zero there, but 0 * NaN is not)
-  else if (swk == 1 && swn >= K && ((swn * esz) % 16) == 0 && aligned(w, 16) && (K % epc) == 0 &&
-           (int64_t)BN * swn * esz + K * esz < (1LL << 31))
-    wp = W_KMAJOR;
+  const int wp = w_path(w, swk, swn, N, K, w_dt);
   const int sw = slim_w(wp, swk, swn);
   if (tile_cfg == nullptr && !gather) slim = pick_slim(M, N, K, w_dt, sw);
   SF_REQUIRE(slim < 0 || sw == S_NMAJOR || sw == S_KMAJOR || (sw >= 0 && slim < SLIM_DMA_ONLY),

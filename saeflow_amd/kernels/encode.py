@@ -69,7 +69,16 @@ def _candidates(w_dtype):
             {"BLOCK_M": 256, "BLOCK_N": 128, "BLOCK_K": bk // 2, "GROUP_M": 4, "NUM_WAVES": 4, "GROUP_N": 0}]
 
 
-def _autotune(key, launch, w_dtype, row_nnz, dev):
+def _default_tiling(M, N, K, W_enc):
+    """The tiling of a call without `config`, as a config: the 256x256 tile, or the small one that the
+    library estimates to be faster for this shape and layout."""
+    got = (ctypes.c_int32 * 6)()
+    _lib.check(_lib.load().sf_encode_tiling(M, N, K, _lib.ptr(W_enc), W_enc.stride(0), W_enc.stride(1),
+                                            _lib.dtype_code(W_enc, "W_enc"), got))
+    return dict(zip(CONFIG_KEYS, got))
+
+
+def _autotune(key, launch, cands, row_nnz, dev):
     """Fastest candidate tiling for `key`. Every candidate is launched once to warm up, then
     timed over AUTOTUNE_ROUNDS interleaved rounds (one launch per candidate per round, so
     clock and power drift spreads over all of them) and ranked by its median; a candidate
@@ -79,9 +88,6 @@ def _autotune(key, launch, w_dtype, row_nnz, dev):
     if key not in _tuned:
         saved = row_nnz.clone() if row_nnz is not None else None
         stream = torch.cuda.current_stream(dev)  # the stream the launches go to
-        # None: the library's own choice, which may be a small tile (ragged shapes, a W_enc whose
-        # rows are not 16-B aligned)
-        cands = [*_candidates(w_dtype), None]
         for cfg in cands:
             launch(cfg)
         events = [[] for _ in cands]
@@ -136,11 +142,13 @@ def _launch(x, W_enc, b_enc, b_dec, threshold, act, out, row_nnz, config):
 
     explicit = config is not None
     if not explicit and AUTOTUNE and 2 * M * N * K >= AUTOTUNE_MIN_FLOPS:
-        key = (M, N, K, x.dtype, W_enc.dtype, out.dtype, W_enc.stride(), act)
-        if torch.cuda.is_current_stream_capturing():
-            config = _tuned.get(key)  # no timing under graph capture: a shape tuned before keeps its pick
-        else:
-            config = _autotune(key, launch, W_enc.dtype, row_nnz, dev)
+        # (the alignment decides how W_enc is staged)
+        key = (M, N, K, x.dtype, W_enc.dtype, out.dtype, W_enc.stride(), W_enc.data_ptr() % 16 == 0, act)
+        config = _tuned.get(key)
+        if config is None and not torch.cuda.is_current_stream_capturing():  # no timing under graph capture
+            cands, own = _candidates(W_enc.dtype), _default_tiling(M, N, K, W_enc)
+            # a small tile (ragged shapes, a W_enc whose rows are not 16-B aligned) is timed with them
+            config = _autotune(key, launch, cands if own in cands else [*cands, own], row_nnz, dev)
     cfg = launch(config)
     if explicit:
         return  # a pinned tiling is not a tuning result: best_config() keeps reporting the last one
@@ -297,7 +305,8 @@ def encode_gather(x, W_enc, b_enc, b_dec, rows, n_rows, threshold=None, activati
 
 def best_config():
     """Tiling chosen by the most recent launch that chose one, i.e. a call without `config`
-    (None until such a call): the autotuner's timed pick for that shape, or the default
-    tiling of a problem too small to time (encode.py:142-144), which stands for the small tile
-    that such a problem may run instead (same bits). Calls that pin `config` leave it unchanged."""
+    (None until such a call): the autotuner's timed pick for that shape, which may be a small tile,
+    or the default tiling of a problem that was not timed (too small, or first met under graph
+    capture; encode.py:142-144), which stands for the small tile that such a problem may run instead
+    (same bits). Calls that pin `config` leave it unchanged."""
     return None if _last_config is None else dict(_last_config)

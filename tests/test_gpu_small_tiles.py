@@ -163,3 +163,31 @@ def test_small_tiles_write_a_strided_output_row_in_place():
                              _lib.ptr(p["b_dec"]), 1, None, 0, _lib.ptr(out), N + 6, 1, 1, None, M, N, K, 0, None,
                              _lib.ptr(ws), ws.numel(), _lib.stream(x.device)))
     assert same(out[:, :N].contiguous(), want) and bool((out[:, N:] == 7.0).all())
+
+
+def test_a_tuned_small_tile_is_reported_and_reproduced_by_its_config():
+    """best_config() after a timed call names what the call keeps, for W_enc rows off 16 B (the small
+    tiles stage those at several times the rate of the others) and on 16 B, which are tuned apart
+    although shape and strides agree."""
+    from saeflow_amd.kernels import best_config
+    from saeflow_amd.kernels import encode as kenc
+    M, K, N, dtype = 1024, 2304, 16384, torch.bfloat16
+    assert 2 * M * N * K >= kenc.AUTOTUNE_MIN_FLOPS
+    x, big, p, _ = make((M, K, N + 8), dtype, "features")
+    be = p["b_enc"][:N]
+    saved = dict(kenc._tuned)
+    kenc._tuned.clear()
+    try:
+        f = fused_encode(x, big[:, :N], be, p["b_dec"])
+        assert best_config() in kenc._candidates(dtype) or best_config()["BLOCK_M"] < 256
+        g = fused_encode(x, big[:, 1:N + 1], be, p["b_dec"])
+        picked = best_config()
+        assert len(kenc._tuned) == 2 and picked["BLOCK_M"] < 256
+        assert picked == kenc._default_tiling(M, N, K, big[:, 1:N + 1])
+        assert same(fused_encode(x, big[:, 1:N + 1], be, p["b_dec"], config=picked), g)
+        fused_encode(x, big[:, :N], be, p["b_dec"])
+        assert best_config() == next(iter(kenc._tuned.values()))  # a shape tuned before keeps its own pick
+        assert same(f, fused_encode(x, big[:, :N].contiguous(), be, p["b_dec"], config=wide(dtype)))
+    finally:
+        kenc._tuned.clear()
+        kenc._tuned.update(saved)

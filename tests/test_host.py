@@ -150,6 +150,25 @@ def test_encode_rows_without_features_still_checks_its_operands():
     assert encode_rows(x[:0], W, torch.zeros(0), b, cap=4)[0].shape == (0,)  # no tokens: nothing to run
 
 
+def _tiling(M, N, K, w=16, swk=None, swn=1, dt=1):
+    got = (ctypes.c_int32 * 6)()
+    _lib.check(_lib.load().sf_encode_tiling(M, N, K, w, N if swk is None else swk, swn, dt, got))
+    return list(got)
+
+
+def test_encode_tiling_names_what_a_call_runs():
+    wide = [256, 256, 64, 1, 8, 8]
+    assert _tiling(16384, 65536, 2304) == wide and _tiling(16384, 65536, 2304, dt=0) == [256, 256, 32, 1, 8, 8]
+    assert _tiling(1, 16384, 2304)[0] == 32  # a token
+    assert _tiling(1, 0, 2304) == wide and _tiling(0, 64, 2304) == wide and _tiling(4, 64, 0) == wide  # no GEMM
+    # rows off 16 B are staged through registers by the small tiles, element by element by 256x256
+    for layout in (dict(w=18), dict(swk=16385), dict(swk=1, swn=2311)):
+        assert _tiling(8192, 16384, 2304, **layout)[0] < 256, layout
+    assert _tiling(8192, 16384, 2304, swk=32768, swn=2) == wide  # strided along both axes
+    assert _lib.load().sf_encode_tiling(1, 1, 1, 16, 1, 1, 7, (ctypes.c_int32 * 6)()) == _lib.SF_EINVAL
+    assert _lib.load().sf_encode_tiling(-1, 1, 1, 16, 1, 1, 1, (ctypes.c_int32 * 6)()) == _lib.SF_EINVAL
+
+
 def test_best_config_is_none_before_a_tuned_launch():
     from saeflow_amd.kernels import best_config
     from saeflow_amd.kernels import encode as kenc
