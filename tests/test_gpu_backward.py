@@ -416,3 +416,65 @@ def test_sparse_backward_takes_vectors_that_are_views():
     got = sparse_backward(xg, sae.W_enc, sae.b_enc, sae.W_dec, spread[3], spread[:3], G, h)
     for name in ("W_enc", "b_enc", "W_dec", "b_dec", "x", "pre"):
         assert torch.equal(getattr(got, name), getattr(want, name)), name
+
+
+@pytest.mark.parametrize("D", [1, 2, 3, 4])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_sparse_backward_with_too_little_dw_enc_for_the_item_records(dtype, D):
+    """A few d_in elements: dW_enc cannot hold the 16-B work-item records (as sf_backward_columns
+    decides), so the plan is walked instead; long, short and unused columns."""
+    import ctypes
+    from saeflow_amd import _lib
+    M, N = 700, 96
+    got, want, (indptr, indices, values) = run_case(M, D, N, "relu", dtype, hot=3)
+    counts = torch.bincount(indices.long(), minlength=N)
+    assert int(counts.max()) == M  # longer than one work item
+    bounds = [ctypes.c_int64() for _ in range(3)]
+    _lib.check(_lib.load().sf_backward_bounds(N, indices.numel(), D, _lib.DTYPE[dtype], *map(ctypes.byref, bounds)))
+    assert D * N * got.W_enc.element_size() < 16 * bounds[0].value
+    for name in ("W_enc", "b_enc", "W_dec", "b_dec", "x"):
+        check(name, getattr(got, name), want[name], dtype)
+
+
+def test_sparse_backward_with_two_of_three_slabs_a_block():
+    """262144 features at d_in 1088 (three 512-element slabs): 4096 column tiles, whose slabs are split
+    over two blocks, the second with one slab (unaligned dW_enc rows too); six slabs in three blocks at
+    131136 features. Closed forms of sampled columns in float64; unused columns exactly zero."""
+    dtype, M = torch.bfloat16, 300
+    for N, D in ((262144, 1088), (262144 - 7, 1088), (131072 + 64, 2600)):
+        g = torch.Generator(device="cuda").manual_seed(N)
+        rand = lambda *sh: torch.randn(*sh, device="cuda", generator=g)  # noqa: E731
+        W_dec, W_enc = rand(N, D).to(dtype), rand(D, N).to(dtype) / 32
+        b_dec, x, G = (0.1 * rand(D)).to(dtype), rand(M, D).to(dtype), rand(M, D).to(dtype)
+        # feature 5 on every row (a heavy column), 64 and N - 1 on some, the others at most a few times
+        cols = torch.randint(200, N, (M, 12), device="cuda", generator=g).sort(1).values
+        cols = torch.cat([torch.full((M, 1), 5, device="cuda"), torch.full((M, 1), 64, device="cuda"), cols,
+                          torch.full((M, 1), N - 1, device="cuda")], 1)
+        keep = torch.ones_like(cols, dtype=torch.bool)
+        keep[:, 1:] = cols[:, 1:] != cols[:, :-1]
+        keep[40:, 1] = False
+        keep[7:, -1] = False
+        indptr = torch.zeros(M + 1, dtype=torch.int64, device="cuda")
+        indptr[1:] = keep.sum(1).cumsum(0)
+        indices = cols[keep].int()
+        values = (rand(indices.numel()).abs() + 0.1).to(dtype)
+        got = sparse_backward(x, W_enc, torch.zeros(N, device="cuda", dtype=dtype), W_dec, b_dec,
+                              (indptr, indices, values), G, need_grad_x=False)
+        rows_of = torch.repeat_interleave(torch.arange(M, device="cuda"), indptr[1:] - indptr[:-1])
+        xs = (x.double() - b_dec.double()).to(dtype).double()
+        want_pre = (G[rows_of].double() * W_dec[indices.long()].double()).sum(1)
+        torch.testing.assert_close(got.pre.double(), want_pre, atol=1e-4 * want_pre.abs().max().item(), rtol=1e-4)
+        counts = torch.bincount(indices.long(), minlength=N)
+        assert int(counts[5]) == M and int(counts[64]) == 40 and int(counts[N - 1]) >= 7
+        used = torch.nonzero(counts).flatten()
+        for j in [5, 64, N - 1, *used[3::used.numel() // 9].tolist()]:
+            sel = indices == j
+            ms, fv, gp = rows_of[sel], values[sel].double(), got.pre[sel].double()
+            check(f"W_dec[{j}]", got.W_dec[j], (fv[:, None] * G[ms].double()).sum(0).cpu(), dtype)
+            check(f"W_enc[:, {j}]", got.W_enc[:, j], (gp[:, None] * xs[ms]).sum(0).cpu(), dtype)
+            check(f"b_enc[{j}]", got.b_enc[j], gp.sum().cpu(), dtype)
+        # of the whole dW_enc: the columns with a nonzero are the used ones, each of full length
+        per_column = sum((got.W_enc[i:i + 256] != 0).sum(0) for i in range(0, D, 256))
+        assert torch.equal(per_column > 0, counts > 0)
+        assert int(per_column[used].min()) > D * 9 // 10
+        assert torch.equal((got.W_dec != 0).any(1), counts > 0) and bool((got.b_enc[counts == 0] == 0).all())
