@@ -134,16 +134,20 @@ __device__ __forceinline__ int64_t block_exclusive_i64(int64_t v, int64_t* s_w, 
   return before + x - v;
 }
 
-// Exclusive prefix over the wave's lanes and wave total of c (0 <= c < 16), from 4 ballots.
-__device__ __forceinline__ void wave_scan16(int c, int lane, int& prefix, int& total) {
+// Exclusive prefix over the wave's lanes and wave total of c (0 <= c < 2^B), from B ballots.
+template <int B>
+__device__ __forceinline__ void wave_scan_bits(int c, int lane, int& prefix, int& total) {
   prefix = 0;
   total = 0;
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {
+  for (int b = 0; b < B; ++b) {
     const uint64_t bal = __ballot((c >> b) & 1);
     prefix += __popcll(bal & lanemask_lt(lane)) << b;
     total += __popcll(bal) << b;
   }
+}
+__device__ __forceinline__ void wave_scan16(int c, int lane, int& prefix, int& total) {
+  wave_scan_bits<4>(c, lane, prefix, total);
 }
 
 // Ascending bitonic sort of the wavefront's 64 * R keys, key r*64 + lane in v[r]: exchanges

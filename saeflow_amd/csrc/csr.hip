@@ -321,10 +321,11 @@ using elem_t = typename std::conditional<ES == 2, u16, uint32_t>::type;
 // of them, in no particular order, in lidx / lval [M, cap], so that a caller without counts reads f once: short
 // rows go from their lists to the CSR (rows_to_csr_wave_kernel), and compact_row_kernel's second pass
 // over f is left to the longer ones, which store no list here. Bound by the one read of f, as
-// count_row_kernel, whose loads and occupancy it keeps: the entries are gathered in LDS, one LDS add per
-// wavefront that holds any until the row is past its list, and stored as one run at the row's end.
-// Measured (us, bf16, 64 nonzeros a row; counts alone / with lists / counts and compaction): 16384 x 65536
-// 304 / 340 / 655, 512 x 2^20 152 / 155 / 323.
+// count_row_kernel, whose loads it keeps: the entries are gathered in LDS, one scan and one LDS add per
+// wavefront and group of loads until the row is past its list, and stored as one run at the row's end.
+// Measured (us, bf16; counts alone / with lists, 64 and 300 nonzeros a row): 16384 x 65536 305 / 336, 312,
+// 16384 x 16384 79 / 89, 83, 512 x 2^20 152 / 155, 154. With a scan and an add per 16-B
+// chunk of each lane the first was 340.
 constexpr int LIST_CAP = 256;
 template <int ES>
 __global__ __launch_bounds__(256) void list_row_kernel(const char* f, int64_t sfm, int64_t N, int cap,
@@ -354,27 +355,33 @@ __global__ __launch_bounds__(256) void list_row_kernel(const char* f, int64_t sf
       const int64_t ch = c0 + u * 256 + t;
       v[u] = __builtin_nontemporal_load((const u32x4*)(rp + (ch < nch ? ch : nch - 1) * 16));
     }
+    uint32_t fl[U];
+    int n = 0;  // this lane's nonzeros of the group
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t ch = c0 + u * 256 + t;
-      const uint32_t fl = ch < nch ? chunk_flags<ES>(v[u]) : 0u;
-      if (__ballot(fl != 0) == 0) continue;  // wave-uniform
-      if (over) {
-        c += __popc(fl);
-        continue;
-      }
-      int pre, tot, base = 0;
-      wave_scan16(__popc(fl), lane, pre, tot);
-      if (lane == 0) base = atomicAdd(&s_n, tot);
-      base = __builtin_amdgcn_readfirstlane(base);
-      over = base + tot > cap;
-      if (fl == 0 || over) continue;
-      int slot = base + pre;
+      fl[u] = c0 + u * 256 + t < nch ? chunk_flags<ES>(v[u]) : 0u;
+      n += __popc(fl[u]);
+    }
+    if (over) {
+      c += n;
+      continue;
+    }
+    if (__ballot(n != 0) == 0) continue;  // wave-uniform
+    int pre, tot, base = 0;
+    wave_scan_bits<EPC == 8 ? 7 : 6>(n, lane, pre, tot);  // n <= U * EPC
+    if (lane == 0) base = atomicAdd(&s_n, tot);
+    base = __builtin_amdgcn_readfirstlane(base);
+    over = base + tot > cap;
+    if (over) continue;
+    int slot = base + pre;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (fl[u] == 0) continue;
       uint32_t mm = chunk_mask<ES>(v[u]);
       while (mm) {
         const int e = __builtin_ctz(mm);
         mm &= mm - 1;
-        put(slot++, ch * EPC + e, chunk_elem_bits<ES>(v[u], e));
+        put(slot++, (c0 + u * 256 + t) * EPC + e, chunk_elem_bits<ES>(v[u], e));
       }
     }
   }

@@ -74,10 +74,14 @@ def compact_into(f, indptr, nnz, longer_than, indices, values):
 
 LIST_CAP = 256  # nonzeros of a row that row_lists keeps: what rows_to_csr sorts in one wavefront
 # dense_to_csr without counts reads f once, through lists, from these sizes on. Measured (us, bf16,
-# counts + compaction -> lists): 16384 x 65536 16 nonzeros a row 641 -> 361, 64 655 -> 388, 200 760 -> 471; 512 x
-# 2^20 64 a row 323 -> 187; 16384 x 16384 209 -> 135, 225 -> 178 at 200 a row. Where every row is longer than its
-# list, the second read comes on top of the lists' work: 300 a row 788 -> 794 (2 GiB of f), 226 -> 237 (512 MiB),
-# 600 a row 812 -> 818 and 236 -> 239. Of smaller f that share grows (f of 64 MiB, 64 a row: 49 either way), so they
+# counts + compaction -> lists): 16384 x 65536 16 nonzeros a row 639 -> 360, 64 655 -> 384, 200 760 -> 450; 512 x
+# 2^20 64 a row 323 -> 185; 16384 x 16384 206 -> 136, 222 -> 178 at 200 a row. Rows past their list are read
+# a second time on top of the lists' work: with 10, 25 and 40% of the rows at 600 and the others at 64 (16384 x
+# 16384) 210 -> 157, 217 -> 173, 222 -> 189; with 256 in the mean, half of them past it, 224 -> 220. Above that
+# it costs up to 2% (265 to 300 a row: 225 -> 230; 16384 x 65536 779 -> 737 at 265, 786 -> 793 at 300; 600 a row 810 ->
+# 812), 3-4% where the chip holds all rows at once (2048 x 131072: 205 -> 212, 208 -> 217, 222 -> 226).
+# Compacting everything as soon as a quarter of the rows is past the list is slower than that: 16384 x
+# 65536 with 40% at 600 603 -> 758. Of smaller f the lists' share grows (f of 64 MiB, 64 a row: 49 either way), so they
 # keep the two passes, as do rows under 32 KiB, where the sort of the lists weighs more (16384 x 4096, 200 a row:
 # 100 -> 113).
 LIST_MIN_BYTES = 1 << 29

@@ -93,3 +93,41 @@ def test_dense_to_csr_of_rows_the_vector_loads_do_not_take(monkeypatch):
         want = g.to_sparse_csr()
         assert torch.equal(indptr, want.crow_indices()) and torch.equal(indices.long(), want.col_indices())
         assert torch.equal(values, want.values())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_dense_to_csr_of_rows_around_the_list_length(dtype, monkeypatch):
+    """Whole 16-B chunks of one thread nonzero (its count of a group of loads is 64 or 32), which fill
+    a row's list exactly or pass it by one; half of the rows past their list; all of them a little past
+    it; and so far past it on average that everything is compacted from f."""
+    monkeypatch.setattr(kernels.decode, "LIST_MIN_BYTES", 0)
+    monkeypatch.setattr(kernels.decode, "LIST_MIN_ROW_BYTES", 0)
+    M, N = 6, 3 * 256 * 8 * 8
+    epc = 8 if dtype == torch.bfloat16 else 4
+
+    def check(f):
+        indptr, indices, values = dense_to_csr(f.cuda())
+        where = (f != 0).nonzero()
+        assert torch.equal(indptr.cpu(), torch.cat([torch.zeros(1, dtype=torch.int64), (f != 0).sum(1).cumsum(0)]))
+        assert torch.equal(indices.cpu(), where[:, 1].int()) and torch.equal(values.cpu(), f[where[:, 0], where[:, 1]])
+
+    f = torch.zeros(M, N, dtype=dtype)
+    for m in range(M):
+        for t in range(256 // (8 * epc)):  # threads of one wavefront, or of several, in the group m // 2
+            for u in range(8):
+                at = ((m // 2) * 2048 + u * 256 + (t if m % 2 else 37 * t % 256)) * epc
+                f[m, at:at + epc] = torch.arange(1, epc + 1).to(dtype) + m
+    assert (f != 0).sum(1).tolist() == [256] * M
+    check(f)
+    f[::2, N - 1] = 1  # every second row passes its list
+    f[1::2, f[1].nonzero()[0]] = 0
+    check(f)
+    f[1::2, N - 2:] = 3
+    check(f)
+    f = torch.zeros(M, N, dtype=dtype)
+    for m in range(M):
+        f[m, torch.randperm(N, generator=torch.Generator().manual_seed(m))[:265 + m]] = 1
+    check(f)
+    f[:, f.sum(0) == 0] = torch.cat([torch.ones(30), torch.zeros(N)])[:int((f.sum(0) == 0).sum())].to(dtype)
+    monkeypatch.setattr(kernels.decode, "rows_to_csr", None)  # 295 and more a row: not sorted at all
+    check(f)
