@@ -70,10 +70,12 @@ def check_encode(got, x, p, activation, dtype):
 def tilings(dtype):
     bk = 32 if dtype == torch.float32 else 64
     return [None, {"BLOCK_M": 256, "BLOCK_N": 128, "BLOCK_K": bk // 2, "GROUP_M": 2},
-            {"BLOCK_M": 256, "BLOCK_N": 256, "BLOCK_K": bk, "GROUP_M": 1, "NUM_WAVES": 4}]
+            {"BLOCK_M": 256, "BLOCK_N": 256, "BLOCK_K": bk, "GROUP_M": 1, "NUM_WAVES": 4},
+            # what None stands for where no small tile is taken
+            {"BLOCK_M": 256, "BLOCK_N": 256, "BLOCK_K": bk}]
 
 
-@pytest.mark.parametrize("narrow", [0, 1, 2])
+@pytest.mark.parametrize("narrow", [0, 1, 2, 3])
 @pytest.mark.parametrize("activation", ["relu", "jumprelu"])
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("shape", SHAPES + VEC_SHAPES)
@@ -216,8 +218,18 @@ def test_fused_encode_strided_weights(dtype):
     x = torch.randn(20, 48).to(dtype)
     q = gpu(p)
     W_t = q["W_enc"].T.contiguous().T
-    got = fused_encode(x.cuda(), W_t, q["b_enc"], q["b_dec"])
-    check_encode(got, x, p, "relu", dtype)
+    for config in (None, tilings(dtype)[3]):
+        got = fused_encode(x.cuda(), W_t, q["b_enc"], q["b_dec"], config=config)
+        check_encode(got, x, p, "relu", dtype)
+    # rows off 16 B (padded with anything): through registers, and element by element on 256x256 tiles
+    wide = torch.full((48, 81), float("nan"), device="cuda", dtype=dtype)
+    wide[:, :80] = q["W_enc"]
+    tall = torch.full((80, 51), float("nan"), device="cuda", dtype=dtype)
+    tall[:, :48] = q["W_enc"].T
+    for W_o in (wide[:, :80], tall[:, :48].T):
+        for config in (None, tilings(dtype)[3]):
+            got = fused_encode(x.cuda(), W_o, q["b_enc"], q["b_dec"], config=config)
+            check_encode(got, x, p, "relu", dtype)
     # arbitrary (non-unit) strides: generic path
     W_s = torch.empty(48, 160, device="cuda", dtype=dtype)[:, ::2]
     W_s.copy_(q["W_enc"])
