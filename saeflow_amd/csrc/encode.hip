@@ -130,6 +130,10 @@ hipError_t launch_slim_dt(const GemmArgs& a, int sw, int shape, int epi, hipStre
   }
 }
 
+// A launch of 2^32 work-items or more is refused by HIP. The slim tiles reach that before the 256x256
+// tile (which has half of the 128x128 tile's work-items per output); such problems keep the latter.
+constexpr int64_t MAX_WORK_ITEMS = UINT32_MAX;
+
 // The slim shape a call without a tile_cfg runs, or -1 for the 256x256 tiles: the smallest of the
 // estimated times below. A tile costs `tile` us of a CU's time once several share it and `alone` us
 // on an idle CU (K-step latencies), both measured on MI355X at d_in 2304 (16-bit) and 768 (fp32) and
@@ -162,6 +166,7 @@ int pick_slim(int64_t M, int64_t N, int64_t K, int w_dt, int sw) {
   for (int i = 0; i < (dma ? SLIM_SHAPES : SLIM_DMA_ONLY); ++i) {
     const SlimShape q = slim_shape(i);
     const int64_t tm = (M + q.tm - 1) / q.tm, tn = (N + q.tn - 1) / q.tn;
+    if (tm * tn * 64 * q.nw > MAX_WORK_ITEMS) continue;
     const Cost c = f32 ? c32[i] : c16[i];
     const double t = estimate(std::max((double)c.alone, tm * tn / cus * c.tile) * scale, tm);
     if (t < least) {
@@ -315,6 +320,8 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
   a.group_m = std::min(group_m, a.tiles_m);
   a.group_n = std::min(group_n, a.tiles_n);
   SF_REQUIRE((int64_t)a.tiles_m * a.tiles_n < (1LL << 31), "%s: too many tiles", fn);
+  SF_REQUIRE(slim < 0 || (int64_t)a.tiles_m * a.tiles_n * 64 * slim_shape(slim).nw <= MAX_WORK_ITEMS,
+             "%s: too many tiles of %dx%d for one launch", fn, tbm, tbn);
   const int oes = sf_dtype_size(out_dt);
   a.vec_store = epi == EPI_DENSE && son == 1 && ((som * oes) % 16) == 0 && aligned(out, 16);
   a.cand_cnt = cand_cnt; a.cand_idx = cand_idx; a.cand_val = (char*)cand_val; a.cap = cap;

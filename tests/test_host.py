@@ -169,6 +169,22 @@ def test_encode_tiling_names_what_a_call_runs():
     assert _lib.load().sf_encode_tiling(-1, 1, 1, 16, 1, 1, 1, (ctypes.c_int32 * 6)()) == _lib.SF_EINVAL
 
 
+def test_small_tiles_whose_grid_one_launch_cannot_hold_are_not_picked():
+    """HIP refuses 2^32 work-items: 262144 tokens of 2^20 - 1 features are 2^32 with 128x128 tiles of 256
+    threads, which a W_enc with rows off 16 B would take; naming such a tile is refused before any launch."""
+    M, N, K = 262144, (1 << 20) - 1, 64
+    for dt in (0, 1, 2):
+        tm, tn, _, _, waves, _ = _tiling(M, N, K, dt=dt)
+        assert -(-M // tm) * -(-N // tn) * 64 * waves < 1 << 32
+        tm, tn, _, _, waves, _ = _tiling(M // 8, N, K, dt=dt)
+        assert tm < 256 and -(-M // 8 // tm) * -(-N // tn) * 64 * waves < 1 << 32
+    lib = _lib.load()
+    cfg = (ctypes.c_int32 * 6)(128, 128, 32, 1, 4, 8)
+    args = (16, K, 1, 1, 16, N, 1, 1, 16, 1, 16, 1, None, 1, None, 16, 16, 16, 1, 8)
+    rc = lib.sf_encode_rows(*args, M, N, K, 0, cfg, 16, 1 << 40, None)
+    assert rc == _lib.SF_EINVAL and b"one launch" in lib.sf_last_error()
+
+
 def test_best_config_is_none_before_a_tuned_launch():
     from saeflow_amd.kernels import best_config
     from saeflow_amd.kernels import encode as kenc
