@@ -68,9 +68,9 @@ SF_API const char* sf_last_error(void);
  *           GROUP_N} naming one of the compiled tilings (encode.py:104 `config=`, whose Triton
  *           configs carry num_warps likewise): {256, 256, BK, G, 8 or 4, GN} or
  *           {256, 128, BK/2, G, 4, GN}, BK = 64 (16-bit W) or 32 (fp32 W), G >= 1, GN >= 0, or,
- *           for a W contiguous along one axis, the small tiles {32 | 64 | 96, 64, BK, G, 2, GN},
+ *           for a W contiguous along one axis, the small tiles {32, 64, BK, G, 2, GN},
  *           {128, 64, BK, G, 4, GN}, {128, 128, BK/2, G, 4, GN}, {32 | 64, 128, BK, G, 4, GN} and
- *           (rows of W 16-B aligned) {128 | 160, 256, BK, G, 4, GN}.
+ *           (rows of W 16-B aligned) {160, 256, BK, G, 4, GN}.
  *           Tile order: GN > 0 walks runs of GN feature tiles, token tile by token tile;
  *           GN = 0 walks runs of G token tiles, feature tile by feature tile (the reference's
  *           GROUP_M order, encode.py:44-52). The order changes speed only, never results.

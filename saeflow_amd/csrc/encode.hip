@@ -149,10 +149,8 @@ int pick_slim(int64_t M, int64_t N, int64_t K, int w_dt, int sw) {
   struct Cost {
     float tile, alone;
   };
-  static constexpr Cost c16[SLIM_SHAPES] = {{7.5f, 9.5f},   {10.5f, 12.5f}, {12.5f, 16.5f}, {14.f, 14.5f}, {23.f, 25.f},
-                                            {10.7f, 12.5f}, {15.f, 14.5f},  {46.f, 36.f},   {44.f, 41.f}};
-  static constexpr Cost c32[SLIM_SHAPES] = {{8.f, 10.f},  {13.7f, 22.f}, {21.f, 34.f},  {24.3f, 24.f}, {47.f, 43.f},
-                                            {13.4f, 14.f}, {24.f, 23.f},  {100.f, 92.f}, {124.f, 115.f}};
+  static constexpr Cost c16[SLIM_SHAPES] = {{7.5f, 9.5f}, {14.f, 14.5f}, {23.f, 25.f}, {10.7f, 12.5f}, {15.f, 14.5f}, {44.f, 41.f}};
+  static constexpr Cost c32[SLIM_SHAPES] = {{8.f, 10.f}, {24.3f, 24.f}, {47.f, 43.f}, {13.4f, 14.f}, {24.f, 23.f}, {124.f, 115.f}};
   const bool f32 = w_dt == SF_F32, dma = sw == S_NMAJOR || sw == S_KMAJOR;
   const double cus = 8 * XCD_CUS, pass = 5.7e6, scale = (double)K / (f32 ? 768 : 2304);
   auto estimate = [&](double mfma, int64_t tiles_m) {
@@ -253,9 +251,9 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
                            tile_cfg[2] == bk / 2 && tile_cfg[4] == 4;
     SF_REQUIRE((is_wide || is_narrow || slim >= 0) && tile_cfg[3] >= 1 && tile_cfg[5] >= 0,
                "%s: unsupported tile config {%d,%d,%d,%d,%d,%d}; compiled tilings: "
-               "{%d,%d,%d,GROUP_M>=1,%d%s,GROUP_N>=0}%s and the small {32|64|96,64,BLOCK_K,G,2,GN}, "
+               "{%d,%d,%d,GROUP_M>=1,%d%s,GROUP_N>=0}%s and the small {32,64,BLOCK_K,G,2,GN}, "
                "{128,64,BLOCK_K,G,4,GN}, {128,128,BLOCK_K/2,G,4,GN}, {32|64,128,BLOCK_K,G,4,GN}, "
-               "{128|160,256,BLOCK_K,G,4,GN}", fn, tile_cfg[0], tile_cfg[1], tile_cfg[2], tile_cfg[3],
+               "{160,256,BLOCK_K,G,4,GN}", fn, tile_cfg[0], tile_cfg[1], tile_cfg[2], tile_cfg[3],
                tile_cfg[4], tile_cfg[5], BM, BN, bk, SF_WIDE_WAVES, epi == EPI_DENSE ? " or 4" : "",
                epi == EPI_DENSE ? " and {256,128,BLOCK_K/2,GROUP_M>=1,4,GROUP_N>=0}" : "");
     group_m = tile_cfg[3];

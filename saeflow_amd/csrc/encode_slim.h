@@ -29,22 +29,18 @@ struct SlimTile {
 // LDS latency of a K-step, which two workgroups per CU overlap (26-36% of the MFMA rate in 16 bits,
 // 87-100% in fp32, against 69% / 95% of a 256x256 tile). Rates at each size beside pick_slim
 // (encode.hip).
-// Up to 32, 64 or 96 tokens: two waves of 32 features each, 128-B W rows, five (three, two) stages
-// in flight and two workgroups per CU.
+// Up to 32 tokens: two waves of 32 features each, 128-B W rows, five stages in flight and two
+// workgroups per CU.
 typedef SlimTile<1, 1, 1, 2, 8, 6> Slim32;
-typedef SlimTile<2, 1, 1, 2, 8, 4> Slim64;
-typedef SlimTile<3, 1, 1, 2, 8, 3> Slim96;
 // 128 tokens: 4 waves of 64 x 32 over a 64-feature panel, or of 64 x 64 over 128 features.
 typedef SlimTile<2, 1, 2, 2, 8, 3> Slim128;
 typedef SlimTile<2, 2, 2, 2, 4, 4> Slim128w;
-// 128- and 256-feature panels (256- and 512-B W rows): one panel (two) per CU at d_sae = 65536.
+// 128-feature panels, and a 256-feature one for up to 160 tokens (256- and 512-B W rows).
 typedef SlimTile<1, 1, 1, 4, 8, 3> Slim32w;
 typedef SlimTile<2, 1, 1, 4, 8, 3> Slim64w;
-typedef SlimTile<4, 2, 1, 4, 8, 3> Slim128x;
 typedef SlimTile<5, 2, 1, 4, 8, 3> Slim160x;
 // Register-staged W: three stages.
 typedef SlimTile<1, 1, 1, 2, 8, 3> Slim32r;
-typedef SlimTile<2, 1, 1, 2, 8, 3> Slim64r;
 typedef SlimTile<2, 2, 2, 2, 4, 3> Slim128wr;
 
 // dma16 with a cache policy: AUX_NT streams past L2, for a W that each launch reads once.
@@ -237,7 +233,7 @@ __global__ __launch_bounds__(TL::NT, TL::ST * TL::NS > 81920 ? TL::NW / 4 : TL::
   constexpr bool NROW = SW == S_NMAJOR || SW == S_NROWS;  // W tile [k][n] in LDS, else [n][k]
   constexpr bool REG = SW == S_NROWS || SW == S_KROWS;
   constexpr int CPR = TN / EPC;  // 16-B chunks per [k][n] row
-  static_assert(NS >= 3 && NS <= 6 && (!REG || NS == 3), "stage buffers");
+  static_assert((NS == 3 || NS == 4 || NS == 6) && (!REG || NS == 3), "stage buffers");
   // distinct LDS objects, so the compiler's wait-count pass can tell the DMA targets from the
   // buffer that fragments are read from
   __shared__ __attribute__((aligned(1024))) char s0[TL::ST];
@@ -526,7 +522,7 @@ __global__ __launch_bounds__(TL::NT, TL::ST * TL::NS > 81920 ? TL::NW / 4 : TL::
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
   for (int kt = 0;;) {  // KT >= 1; the buffers (and the W register sets) rotate statically
-    step(S0{}, kt, s0, NS == 3 ? s2 : (NS == 4 ? s3 : (NS == 5 ? s4 : s5)), s1);
+    step(S0{}, kt, s0, NS == 3 ? s2 : (NS == 4 ? s3 : s5), s1);
     if (++kt >= KT) break;
     step(S1{}, kt, s1, s0, s2);
     if (++kt >= KT) break;
@@ -545,7 +541,7 @@ __global__ __launch_bounds__(TL::NT, TL::ST * TL::NS > 81920 ? TL::NW / 4 : TL::
       if (++kt >= KT) break;
     }
     if constexpr (NS > 4) {
-      step(S0{}, kt, s4, s3, NS == 5 ? s0 : s5);
+      step(S0{}, kt, s4, s3, s5);
       if (++kt >= KT) break;
     }
     if constexpr (NS > 5) {
@@ -569,7 +565,7 @@ __global__ __launch_bounds__(TL::NT, TL::ST * TL::NS > 81920 ? TL::NW / 4 : TL::
 }
 
 // The compiled shapes, by index (sf_encode's tile_cfg names them by BLOCK_M x BLOCK_N).
-constexpr int SLIM_SHAPES = 9, SLIM_DMA_ONLY = 7;  // from SLIM_DMA_ONLY on: no register-staged W
+constexpr int SLIM_SHAPES = 6, SLIM_DMA_ONLY = 5;  // from SLIM_DMA_ONLY on: no register-staged W
 struct SlimShape {
   int tm, tn, kc, nw;
 };
@@ -579,8 +575,8 @@ constexpr SlimShape slim_shape_of() {
 }
 constexpr SlimShape slim_shape(int i) {
   constexpr SlimShape all[SLIM_SHAPES] = {
-      slim_shape_of<Slim32>(),  slim_shape_of<Slim64>(),  slim_shape_of<Slim96>(),  slim_shape_of<Slim128>(), slim_shape_of<Slim128w>(),
-      slim_shape_of<Slim32w>(), slim_shape_of<Slim64w>(), slim_shape_of<Slim128x>(), slim_shape_of<Slim160x>()};
+      slim_shape_of<Slim32>(),  slim_shape_of<Slim128>(), slim_shape_of<Slim128w>(),
+      slim_shape_of<Slim32w>(), slim_shape_of<Slim64w>(), slim_shape_of<Slim160x>()};
   return all[i];
 }
 
@@ -608,15 +604,13 @@ hipError_t launch_slim(const GemmArgs& a, int shape, int epi, hipStream_t s) {
   constexpr bool REG = SW == S_NROWS || SW == S_KROWS;
   switch (shape) {
     case 0: return launch_slim_tile<DT, SW, std::conditional_t<REG, Slim32r, Slim32>>(a, epi, s);
-    case 1: return launch_slim_tile<DT, SW, std::conditional_t<REG, Slim64r, Slim64>>(a, epi, s);
-    case 2: return launch_slim_tile<DT, SW, Slim96>(a, epi, s);
-    case 3: return launch_slim_tile<DT, SW, Slim128>(a, epi, s);
-    case 4: return launch_slim_tile<DT, SW, std::conditional_t<REG, Slim128wr, Slim128w>>(a, epi, s);
-    case 5: return launch_slim_tile<DT, SW, Slim32w>(a, epi, s);
-    case 6: return launch_slim_tile<DT, SW, Slim64w>(a, epi, s);
+    case 1: return launch_slim_tile<DT, SW, Slim128>(a, epi, s);
+    case 2: return launch_slim_tile<DT, SW, std::conditional_t<REG, Slim128wr, Slim128w>>(a, epi, s);
+    case 3: return launch_slim_tile<DT, SW, Slim32w>(a, epi, s);
+    case 4: return launch_slim_tile<DT, SW, Slim64w>(a, epi, s);
     default: break;
   }
-  if constexpr (!REG) return shape == 7 ? launch_slim_tile<DT, SW, Slim128x>(a, epi, s) : launch_slim_tile<DT, SW, Slim160x>(a, epi, s);
+  if constexpr (!REG) return launch_slim_tile<DT, SW, Slim160x>(a, epi, s);
   return hipErrorInvalidValue;
 }
 #endif

@@ -172,8 +172,8 @@ def fused_encode(x, W_enc, b_enc, b_dec, threshold=None, activation="relu", *,
     config: dict {BLOCK_M, BLOCK_N, BLOCK_K, GROUP_M, NUM_WAVES, GROUP_N} naming a compiled
       tiling: {256, 256, 64 (32 for fp32), G, 8 or 4, GN} (256x256 tiles of 8 waves of 128x64
       or 4 waves of 128x128) or {256, 128, 32 (16), G, 4, GN} (two workgroups per CU), or a small
-      tile {32 | 64 | 96, 64, 64 (32), G, 2, GN}, {128, 64, 64 (32), G, 4, GN}, {128, 128, 32 (16),
-      G, 4, GN}, {32 | 64, 128, 64 (32), G, 4, GN}, {128 | 160, 256, 64 (32), G, 4, GN}, and its
+      tile {32, 64, 64 (32), G, 2, GN}, {128, 64, 64 (32), G, 4, GN}, {128, 128, 32 (16),
+      G, 4, GN}, {32 | 64, 128, 64 (32), G, 4, GN}, {160, 256, 64 (32), G, 4, GN}, and its
       tile order: runs of GN feature tiles if GN > 0, else runs of G token tiles (GN 0, the
       default of a dict without it); None = autotuned, or, for problems too small to time, the
       256x256 tile or a small one by an estimate of both.
