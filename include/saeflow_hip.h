@@ -123,11 +123,11 @@ SF_API int sf_encode_workspace_size(int64_t M, int64_t K, int w_dt, int64_t* byt
  * best_config() (encode.py:142-144), which reports the autotuner's pick. */
 SF_API int sf_encode_config(int64_t M, int64_t N, int64_t K, int w_dt, int32_t* cfg_out);
 
-/* Tiling that sf_encode and sf_encode_rows run without a tile_cfg for a W at this address and with these
- * strides (W is not read), as sf_encode_config writes it: the default or a small tile. Naming it as the
- * tile_cfg runs the same kernel. */
+/* Tiling that sf_encode (rows 0) or sf_encode_rows (rows 1) runs without a tile_cfg for a W at this address
+ * and with these strides (W is not read), as sf_encode_config writes it: the default or a small tile.
+ * Naming it as the tile_cfg runs the same kernel. */
 SF_API int sf_encode_tiling(int64_t M, int64_t N, int64_t K, const void* w, int64_t swk, int64_t swn, int w_dt,
-                     int32_t* cfg_out);
+                     int rows, int32_t* cfg_out);
 
 /*
  * Row-candidate encode: the fused encode without the dense output. Each row's kept values

@@ -33,7 +33,7 @@ SIGNATURES = {
                                  _P, _I64, _I64, _I32, _P, _I64, _I64, _I64, _I32, _P, _P]),
     "sf_encode_workspace_size": (_I32, [_I64, _I64, _I32, _P]),
     "sf_encode_config": (_I32, [_I64, _I64, _I64, _I32, _P]),
-    "sf_encode_tiling": (_I32, [_I64, _I64, _I64, _P, _I64, _I64, _I32, _P]),
+    "sf_encode_tiling": (_I32, [_I64, _I64, _I64, _P, _I64, _I64, _I32, _I32, _P]),
     "sf_encode_rows": (_I32, [_P, _I64, _I64, _I32, _P, _I64, _I64, _I32, _P, _I32, _P, _I32, _P, _I32, _P,
                               _P, _P, _P, _I32, _I64, _I64, _I64, _I64, _I32, _P, _P, _I64, _P]),
     "sf_encode_rows_cleared": (_I32, [_P, _I64, _I64, _I32, _P, _I64, _I64, _I32, _P, _I32, _P, _I32, _P, _I32, _P,

@@ -134,39 +134,70 @@ hipError_t launch_slim_dt(const GemmArgs& a, int sw, int shape, int epi, hipStre
 // tile (which has half of the 128x128 tile's work-items per output); such problems keep the latter.
 constexpr int64_t MAX_WORK_ITEMS = UINT32_MAX;
 
-// The slim shape a call without a tile_cfg runs, or -1 for the 256x256 tiles: the smallest of the
-// estimated times below. A tile costs `tile` us of a CU's time once several share it and `alone` us
-// on an idle CU (K-step latencies), both measured on MI355X at d_in 2304 (16-bit) and 768 (fp32) and
-// proportional to d_in; slim tiles of a CU overlap, 256x256 tiles come in whole rounds. A call with
-// one token tile is also one pass over W at `pass` bytes per us, which hides most of the shorter of
-// the two. Measured (us a call, both sides with the x' launch): bf16 d_in 2304 d_sae 16384, 1 token
-// 53 -> 21 (32x64), 137 tokens 54 -> 30, 384 tokens 55 -> 47, from 512 tokens on 256x256 wins; d_sae
-// 65536, 1 token 63 -> 53 (32x128), 137 tokens row lists 102 -> 87 (160x256); fp32 d_in 768, 1 token
-// of d_sae 12288 185 -> 23, 300 tokens 187 -> 57; an odd d_sae of 10007, d_in 1000, 1000 tokens 143
-// (element-wise staging) -> 57.
-int pick_slim(int64_t M, int64_t N, int64_t K, int w_dt, int sw) {
+// The slim shape a call without a tile_cfg runs, or -1 for the 256x256 tiles: the least of the
+// estimated times (us) of the GEMM launch.
+//   slim: a CU with n tiles takes (alone^4 + (n tile)^4)^(1/4): the K-step latencies of one tile, then
+//     the rate of several sharing the CU. n is the mean over the CUs, drawn towards the fullest CU, and
+//     whole rounds for the 160x256 tile, which has a CU to itself. The pass over W runs at `pass` TB/s
+//     (W again from the caches for each further token tile) and hides most of the shorter of the two.
+//   256x256: whole rounds of `tile`; a round that fills the chip in part is nearer to `alone`. Its pass
+//     over W, with one token tile, hides the rest or is hidden.
+//   Both: `fixed`, and `out` a million outputs; of row lists those of 160 tokens, as what they cost is
+//     the queue of atomics on a row's count.
+// The constants are fitted to measured times and to the picks that they lead to, dense and row lists: 3281
+// shapes in 16 bits (d_in 64 to 4096, d_sae 1024 to 140000, 1 to 8192 tokens), 1173 in fp32, 1296 with rows
+// off 16 B. Picks over 2% slower than 256x256: 40 of 6563 in 16 bits, 3 of 2346 in fp32, 15% at most; mean
+// time against 256x256 alone 0.68 (dense), 0.72 (row lists), 0.27 (fp32), and 1.01 of each shape's best tile.
+// An estimate without the partial rounds of 256x256, the fixed parts and a difference between dense and
+// row lists lost over 2% in 755 of the 6563: bf16 d_in 1024, 1280 tokens of d_sae 16384 56 -> 66 us, 512 tokens
+// 28 -> 34, d_in 768 2048 tokens of 4096 26 -> 31. Now, us with the x' launch, 256x256 / pick: bf16 d_in 2304
+// d_sae 16384, 1 token 46 / 18, 128 tokens 46 / 22, 320 tokens 49 / 42, from 385 on 256x256; d_sae 65536, 160
+// tokens as row lists 106 / 94; fp32 d_in 768 d_sae 12288, 300 tokens 185 / 60; rows off 16 B, bf16 d_in 2304,
+// 16385 features, 128 tokens 248 / 36.
+struct Cost {
+  float tile, alone, pass, fixed, out;
+};
+int pick_slim(int64_t M, int64_t N, int64_t K, int w_dt, int sw, bool rows) {
   if (sw < 0 || K == 0) return -1;
-  struct Cost {
-    float tile, alone;
-  };
-  static constexpr Cost c16[SLIM_SHAPES] = {{7.5f, 9.5f}, {14.f, 14.5f}, {23.f, 25.f}, {10.7f, 12.5f}, {15.f, 14.5f}, {44.f, 41.f}};
-  static constexpr Cost c32[SLIM_SHAPES] = {{8.f, 10.f}, {24.3f, 24.f}, {47.f, 43.f}, {13.4f, 14.f}, {24.f, 23.f}, {124.f, 115.f}};
+  enum { DMA16, DMA16_ROWS, REG16, DMA32, REG32 };
+  static constexpr Cost costs[5][SLIM_SHAPES] = {
+      {{6.1f, 6.5f, 6.3f, 3.7f, 1.38f}, {12.2f, 11.5f, 5.f, 6.4f, 0.65f}, {14.5f, 21.7f, 5.f, 4.3f, 1.99f},
+       {9.4f, 11.7f, 7.1f, 3.6f, 1.04f}, {12.6f, 13.6f, 7.f, 5.2f, 0.38f}, {40.9f, 0.f, 7.2f, 8.5f, 7.51f}},
+      {{5.3f, 6.3f, 7.f, 7.9f, 3.52f}, {10.2f, 11.5f, 4.f, 9.2f, 1.64f}, {13.3f, 27.3f, 8.2f, 8.4f, 1.53f},
+       {8.1f, 10.8f, 7.9f, 7.4f, 3.95f}, {10.5f, 10.7f, 6.7f, 12.7f, 1.37f}, {35.6f, 0.f, 14.1f, 14.5f, 1.6f}},
+      {{12.6f, 20.8f, 5.6f, 11.f, 2.76f}, {16.8f, 20.3f, 4.4f, 12.f, 1.58f}, {24.7f, 33.7f, 5.3f, 12.3f, 1.47f},
+       {13.f, 35.7f, 5.6f, 11.2f, 2.75f}, {15.f, 31.7f, 5.5f, 13.3f, 1.96f}},
+      {{8.f, 12.6f, 6.4f, 8.9f, 3.81f}, {21.7f, 19.4f, 7.5f, 8.8f, 4.87f}, {41.1f, 32.6f, 14.3f, 10.1f, 2.09f},
+       {11.4f, 18.5f, 6.8f, 8.2f, 2.39f}, {20.4f, 23.1f, 7.9f, 8.9f, 2.26f}, {104.5f, 0.f, 14.f, 14.9f, 6.15f}},
+      {{11.5f, 24.f, 4.6f, 9.8f, 3.54f}, {28.8f, 22.4f, 13.7f, 11.4f, 1.f}, {55.8f, 47.6f, 12.9f, 13.8f, 0.55f},
+       {18.f, 25.6f, 12.9f, 9.7f, 2.f}, {29.6f, 33.f, 14.f, 11.7f, 0.96f}}};
+  static constexpr Cost wide[5] = {{50.4f, 42.6f, 12.2f, 5.6f, 0.35f}, {30.6f, 39.9f, 5.4f, 7.9f, 2.f}, {},
+                                   {151.1f, 160.8f, 12.1f, 16.3f, 2.04f}, {}};
   const bool f32 = w_dt == SF_F32, dma = sw == S_NMAJOR || sw == S_KMAJOR;
-  const double cus = 8 * XCD_CUS, pass = 5.7e6, scale = (double)K / (f32 ? 768 : 2304);
-  auto estimate = [&](double mfma, int64_t tiles_m) {
-    const double bytes = tiles_m == 1 ? (double)N * K * sf_dtype_size(w_dt) / pass : 0;
-    return std::max(mfma, bytes) + 0.25 * std::min(mfma, bytes);
-  };
-  const int64_t wm = (M + BM - 1) / BM, wn = (N + BN - 1) / BN;
+  const int kind = f32 ? (dma ? DMA32 : REG32) : (dma ? (rows ? DMA16_ROWS : DMA16) : REG16);
+  const double cus = 8 * XCD_CUS, scale = (double)K / (f32 ? 768 : 2304), mb = 1e-6 * N * K * sf_dtype_size(w_dt);
+  const double outs = 1e-6 * N * (kind == DMA16_ROWS ? std::min<int64_t>(M, 160) : M);
+  auto pow4 = [](double v) { return v * v * v * v; };
+  double least = 1e300;  // (a W staged element by element: never the 256x256 tiles)
+  if (dma) {
+    const Cost& c = wide[kind];
+    const int64_t tm = (M + BM - 1) / BM;
+    const double n = (double)tm * ((N + BN - 1) / BN) / cus, full = std::ceil(n) - 1;
+    const double mfma = (full * c.tile + c.alone + (c.tile - c.alone) * pow4(n - full)) * scale;
+    least = std::max(mfma, tm == 1 ? mb / c.pass : 0) + c.fixed + c.out * outs;
+    if (!rows && N % (16 / sf_dtype_size(w_dt)) != 0) least += 1.1e-6 * M * N;  // output rows off 16 B
+  }
   int best = -1;
-  // (a W staged element by element: never the 256x256 tiles)
-  double least = dma ? estimate(std::ceil(wm * wn / cus) * (f32 ? 173 : 45) * scale, wm) : 1e300;
   for (int i = 0; i < (dma ? SLIM_SHAPES : SLIM_DMA_ONLY); ++i) {
     const SlimShape q = slim_shape(i);
+    const Cost& c = costs[kind][i];
     const int64_t tm = (M + q.tm - 1) / q.tm, tn = (N + q.tn - 1) / q.tn;
     if (tm * tn * 64 * q.nw > MAX_WORK_ITEMS) continue;
-    const Cost c = f32 ? c32[i] : c16[i];
-    const double t = estimate(std::max((double)c.alone, tm * tn / cus * c.tile) * scale, tm);
+    const double mean = (double)tm * tn / cus, most = std::ceil(mean);
+    const double n = q.tn == 256 ? most : 0.25 * mean + 0.75 * most;
+    const double mfma = std::sqrt(std::sqrt(pow4(c.alone) + pow4(n * c.tile))) * scale;
+    const double w = mb / c.pass * (1 + 0.1 * (tm - 1));
+    const double t = std::max(mfma, w) + 0.25 * std::min(mfma, w) + c.fixed + c.out * outs;
     if (t < least) {
       least = t;
       best = i;
@@ -178,11 +209,11 @@ int pick_slim(int64_t M, int64_t N, int64_t K, int w_dt, int sw) {
 }  // namespace
 
 extern "C" int sf_encode_tiling(int64_t M, int64_t N, int64_t K, const void* w, int64_t swk, int64_t swn, int w_dt,
-                                int32_t* cfg_out) {
+                                int rows, int32_t* cfg_out) {
   const int rc = sf_encode_config(M, N, K, w_dt, cfg_out);
   if (rc != SF_OK) return rc;
   SF_REQUIRE(M >= 0 && N >= 0 && K >= 0, "sf_encode_tiling: negative size");
-  const int i = M == 0 || N == 0 ? -1 : pick_slim(M, N, K, w_dt, slim_w(w_path(w, swk, swn, N, K, w_dt), swk, swn));
+  const int i = M == 0 || N == 0 ? -1 : pick_slim(M, N, K, w_dt, slim_w(w_path(w, swk, swn, N, K, w_dt), swk, swn), rows != 0);
   if (i >= 0) {
     const SlimShape q = slim_shape(i);
     cfg_out[0] = q.tm;
@@ -297,7 +328,7 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
 
   const int wp = w_path(w, swk, swn, N, K, w_dt);
   const int sw = slim_w(wp, swk, swn);
-  if (tile_cfg == nullptr && !gather) slim = pick_slim(M, N, K, w_dt, sw);
+  if (tile_cfg == nullptr && !gather) slim = pick_slim(M, N, K, w_dt, sw, epi != EPI_DENSE);
   SF_REQUIRE(slim < 0 || sw == S_NMAJOR || sw == S_KMAJOR || (sw >= 0 && slim < SLIM_DMA_ONLY),
              "%s: the small tilings need W contiguous along one axis (those of 256 features also 16-B aligned rows)", fn);
 

@@ -74,7 +74,7 @@ def _default_tiling(M, N, K, W_enc):
     library estimates to be faster for this shape and layout."""
     got = (ctypes.c_int32 * 6)()
     _lib.check(_lib.load().sf_encode_tiling(M, N, K, _lib.ptr(W_enc), W_enc.stride(0), W_enc.stride(1),
-                                            _lib.dtype_code(W_enc, "W_enc"), got))
+                                            _lib.dtype_code(W_enc, "W_enc"), 0, got))
     return dict(zip(CONFIG_KEYS, got))
 
 

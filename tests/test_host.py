@@ -150,9 +150,9 @@ def test_encode_rows_without_features_still_checks_its_operands():
     assert encode_rows(x[:0], W, torch.zeros(0), b, cap=4)[0].shape == (0,)  # no tokens: nothing to run
 
 
-def _tiling(M, N, K, w=16, swk=None, swn=1, dt=1):
+def _tiling(M, N, K, w=16, swk=None, swn=1, dt=1, rows=0):
     got = (ctypes.c_int32 * 6)()
-    _lib.check(_lib.load().sf_encode_tiling(M, N, K, w, N if swk is None else swk, swn, dt, got))
+    _lib.check(_lib.load().sf_encode_tiling(M, N, K, w, N if swk is None else swk, swn, dt, rows, got))
     return list(got)
 
 
@@ -165,8 +165,21 @@ def test_encode_tiling_names_what_a_call_runs():
     for layout in (dict(w=18), dict(swk=16385), dict(swk=1, swn=2311)):
         assert _tiling(8192, 16384, 2304, **layout)[0] < 256, layout
     assert _tiling(8192, 16384, 2304, swk=32768, swn=2) == wide  # strided along both axes
-    assert _lib.load().sf_encode_tiling(1, 1, 1, 16, 1, 1, 7, (ctypes.c_int32 * 6)()) == _lib.SF_EINVAL
-    assert _lib.load().sf_encode_tiling(-1, 1, 1, 16, 1, 1, 1, (ctypes.c_int32 * 6)()) == _lib.SF_EINVAL
+    assert _lib.load().sf_encode_tiling(1, 1, 1, 16, 1, 1, 7, 0, (ctypes.c_int32 * 6)()) == _lib.SF_EINVAL
+    assert _lib.load().sf_encode_tiling(-1, 1, 1, 16, 1, 1, 1, 0, (ctypes.c_int32 * 6)()) == _lib.SF_EINVAL
+
+
+@pytest.mark.parametrize("M,N,K,rows,tile", [
+    # measured more than 10% slower on a small tile than on 256x256
+    (1280, 16384, 1024, 0, 256), (512, 16384, 1024, 0, 256), (512, 16384, 2304, 0, 256), (448, 16384, 2304, 0, 256),
+    (2048, 4096, 768, 0, 256), (256, 32768, 2304, 0, 256), (192, 32768, 2304, 0, 256), (320, 24576, 768, 0, 256),
+    (128, 65536, 2304, 0, 256), (300, 40000, 512, 0, 256),
+    # measured at least 10% faster on this one
+    (1, 16384, 2304, 1, 32), (137, 65536, 2304, 1, 160), (256, 16384, 2304, 0, 64), (128, 24576, 768, 0, 64),
+])
+def test_tile_picks_at_measured_shapes(M, N, K, rows, tile):
+    for dt in (1, 2):
+        assert _tiling(M, N, K, dt=dt, rows=rows)[0] == tile
 
 
 def test_small_tiles_whose_grid_one_launch_cannot_hold_are_not_picked():
@@ -174,10 +187,11 @@ def test_small_tiles_whose_grid_one_launch_cannot_hold_are_not_picked():
     threads, which a W_enc with rows off 16 B would take; naming such a tile is refused before any launch."""
     M, N, K = 262144, (1 << 20) - 1, 64
     for dt in (0, 1, 2):
-        tm, tn, _, _, waves, _ = _tiling(M, N, K, dt=dt)
-        assert -(-M // tm) * -(-N // tn) * 64 * waves < 1 << 32
-        tm, tn, _, _, waves, _ = _tiling(M // 8, N, K, dt=dt)
-        assert tm < 256 and -(-M // 8 // tm) * -(-N // tn) * 64 * waves < 1 << 32
+        for rows in (0, 1):
+            tm, tn, _, _, waves, _ = _tiling(M, N, K, dt=dt, rows=rows)
+            assert -(-M // tm) * -(-N // tn) * 64 * waves < 1 << 32
+            tm, tn, _, _, waves, _ = _tiling(M // 8, N, K, dt=dt, rows=rows)
+            assert tm < 256 and -(-M // 8 // tm) * -(-N // tn) * 64 * waves < 1 << 32
     lib = _lib.load()
     cfg = (ctypes.c_int32 * 6)(128, 128, 32, 1, 4, 8)
     args = (16, K, 1, 1, 16, N, 1, 1, 16, 1, 16, 1, None, 1, None, 16, 16, 16, 1, 8)
