@@ -106,9 +106,10 @@ int w_path(const void* w, int64_t swk, int64_t swn, int64_t N, int64_t K, int w_
       (int64_t)bk * swk * esz + N * esz < (1LL << 31))
     return W_NMAJOR;
   // (K in whole 16-B chunks: a chunk that straddles K would bring in what lies behind the row, its
-  // padding or a parent tensor's columns; x' is zero there, but 0 * NaN is not)
+  // padding or a parent tensor's columns; x' is zero there, but 0 * NaN is not. A tile's rows within
+  // OOB bytes: chunks past K are read at that offset, to come in as zeros.)
   if (swk == 1 && swn >= K && ((swn * esz) % 16) == 0 && aligned(w, 16) && (K % epc) == 0 &&
-      (int64_t)BN * swn * esz + K * esz < (1LL << 31))
+      (int64_t)BN * swn * esz + K * esz <= (int64_t)OOB)
     return W_KMAJOR;
   return W_GENERIC;
 }
@@ -327,7 +328,8 @@ int encode_impl(const char* fn, int epi, const void* x, int64_t sxm, int64_t sxk
   a.row_nnz = row_nnz; a.M = M; a.N = N; a.K = K; a.act = act;
 
   const int wp = w_path(w, swk, swn, N, K, w_dt);
-  const int sw = slim_w(wp, swk, swn);
+  // (d_in = 0: nothing to read, which the register staging, clamped to a last row, cannot express)
+  const int sw = K > 0 ? slim_w(wp, swk, swn) : S_KMAJOR;
   if (tile_cfg == nullptr && !gather) slim = pick_slim(M, N, K, w_dt, sw, epi != EPI_DENSE);
   SF_REQUIRE(slim < 0 || sw == S_NMAJOR || sw == S_KMAJOR || (sw >= 0 && slim < SLIM_DMA_ONLY),
              "%s: the small tilings need W contiguous along one axis (those of 256 features also 16-B aligned rows)", fn);

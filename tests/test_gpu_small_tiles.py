@@ -116,6 +116,18 @@ def test_padding_behind_d_in_stays_out_of_the_features(dtype, d_in):
         assert same(f[:, :N].contiguous(), want), c
 
 
+def test_rows_of_w_enc_megabytes_apart():
+    """A view of d_in 8 into rows of 4 MB and more, NaN behind it: a tile's 256 features span over 1 GiB, the
+    offset that stands for out of range in the DMA path."""
+    M, K, N, pitch = 40, 8, 300, (1 << 21) + (1 << 15)
+    back = torch.full((N, pitch), float("nan"), dtype=torch.bfloat16, device="cuda")
+    x, W, p, _ = make((M, K, N), torch.bfloat16, "features")
+    back[:, :K] = W.T
+    want = fused_encode(x, W, p["b_enc"], p["b_dec"], config=wide(torch.bfloat16))
+    for c in (None, wide(torch.bfloat16), config((32, 64, 2), torch.bfloat16)):
+        assert same(fused_encode(x, back[:, :K].T, p["b_enc"], p["b_dec"], config=c), want), c
+
+
 @pytest.mark.parametrize("tile", TILES)
 @pytest.mark.parametrize("layout", ["features", "odd_features"])
 @pytest.mark.parametrize("dtype", DTYPES)

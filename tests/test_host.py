@@ -162,7 +162,7 @@ def test_encode_tiling_names_what_a_call_runs():
     assert _tiling(1, 16384, 2304)[0] == 32  # a token
     assert _tiling(1, 0, 2304) == wide and _tiling(0, 64, 2304) == wide and _tiling(4, 64, 0) == wide  # no GEMM
     # rows off 16 B are staged through registers by the small tiles, element by element by 256x256
-    for layout in (dict(w=18), dict(swk=16385), dict(swk=1, swn=2311)):
+    for layout in (dict(w=18), dict(swk=16385), dict(swk=1, swn=2311), dict(swk=1, swn=(1 << 21) + 8)):
         assert _tiling(8192, 16384, 2304, **layout)[0] < 256, layout
     assert _tiling(8192, 16384, 2304, swk=32768, swn=2) == wide  # strided along both axes
     assert _lib.load().sf_encode_tiling(1, 1, 1, 16, 1, 1, 7, 0, (ctypes.c_int32 * 6)()) == _lib.SF_EINVAL
